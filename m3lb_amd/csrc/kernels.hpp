@@ -1094,6 +1094,43 @@ __device__ __forceinline__ unsigned interior_id(const Dom& d, int x, int y, int 
   return unsigned(((z + d.hz) * d.sy + (y + d.hy)) * d.sx + x + d.hx);
 }
 
+// Finite-difference gradient grad[a][b] = d_a u_b at a corner node
+// (FluidSolver.hpp:952-998): one-sided where the box ends, central elsewhere.
+// vel_at(r, x, y, z, out) is the velocity at a stencil node, r its place in the
+// node's list of reads.
+template <class K, class VelAt>
+__device__ __forceinline__ void corner_gradient(const Dom& d, int x, int y, int z,
+                                                const typename K::R* uw, VelAt&& vel_at,
+                                                typename K::R grad[3][3]) {
+  using R = typename K::R;
+  const int ic[3] = {x, y, z}, nn[3] = {d.nx, d.ny, d.nz}, per[3] = {d.px, d.py, d.pz};
+  for (int a = 0; a < 3; ++a)
+    for (int b = 0; b < 3; ++b) grad[a][b] = R(0);
+  for (int ax = 0; ax < K::D; ++ax) {
+    if (nn[ax] < 3) continue;
+    int dir = 0;
+    if (!per[ax]) {
+      if (ic[ax] == 0) dir = 1;
+      else if (ic[ax] == nn[ax] - 1) dir = -1;
+    }
+    int c1[3] = {ic[0], ic[1], ic[2]}, c2[3] = {ic[0], ic[1], ic[2]};
+    R u1[3], u2[3];
+    if (dir != 0) {
+      c1[ax] += dir; c2[ax] += 2 * dir;
+      vel_at(2 * ax, c1[0], c1[1], c1[2], u1);
+      vel_at(2 * ax + 1, c2[0], c2[1], c2[2], u2);
+      for (int b = 0; b < K::D; ++b)
+        grad[ax][b] = R(dir) * (R(-1.5) * uw[b] + R(2) * u1[b] - R(0.5) * u2[b]);
+    } else {
+      c1[ax] = (ic[ax] + 1) % nn[ax];
+      c2[ax] = (ic[ax] - 1 + nn[ax]) % nn[ax];
+      vel_at(2 * ax, c1[0], c1[1], c1[2], u1);
+      vel_at(2 * ax + 1, c2[0], c2[1], c2[2], u2);
+      for (int b = 0; b < K::D; ++b) grad[ax][b] = R(0.5) * (u1[b] - u2[b]);
+    }
+  }
+}
+
 // corner_density<P>, first half: rho of every straight-wall node (imposed at
 // the outflow codes).
 template <class K, int P>
@@ -1258,8 +1295,6 @@ __global__ void __launch_bounds__(kBlock) k_walls(WallArgs a) {
   }
   if (collide_it) {
     if (a.fd_corners && code == kNrmCorner) {
-      const int ic[3] = {x, y, z}, nn[3] = {d.nx, d.ny, d.nz}, per[3] = {d.px, d.py, d.pz};
-      R grad[3][3] = {{R(0), R(0), R(0)}, {R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
       // velocity at a stencil node: imposed (table) at a wall node, else from
       // its incoming set
       auto vel_at = [&](int r, int cx, int cy, int cz, R out[3]) {
@@ -1272,29 +1307,8 @@ __global__ void __launch_bounds__(kBlock) k_walls(WallArgs a) {
         incoming(r, m, g);
         set_velocity<K>(g, out, false);
       };
-      for (int ax = 0; ax < K::D; ++ax) {
-        if (nn[ax] < 3) continue;
-        int dir = 0;
-        if (!per[ax]) {
-          if (ic[ax] == 0) dir = 1;
-          else if (ic[ax] == nn[ax] - 1) dir = -1;
-        }
-        int c1[3] = {ic[0], ic[1], ic[2]}, c2[3] = {ic[0], ic[1], ic[2]};
-        R u1[3], u2[3];
-        if (dir != 0) {
-          c1[ax] += dir; c2[ax] += 2 * dir;
-          vel_at(2 * ax, c1[0], c1[1], c1[2], u1);
-          vel_at(2 * ax + 1, c2[0], c2[1], c2[2], u2);
-          for (int b = 0; b < K::D; ++b)
-            grad[ax][b] = R(dir) * (R(-1.5) * uw[b] + R(2) * u1[b] - R(0.5) * u2[b]);
-        } else {
-          c1[ax] = (ic[ax] + 1) % nn[ax];
-          c2[ax] = (ic[ax] - 1 + nn[ax]) % nn[ax];
-          vel_at(2 * ax, c1[0], c1[1], c1[2], u1);
-          vel_at(2 * ax + 1, c2[0], c2[1], c2[2], u2);
-          for (int b = 0; b < K::D; ++b) grad[ax][b] = R(0.5) * (u1[b] - u2[b]);
-        }
-      }
+      R grad[3][3];
+      corner_gradient<K>(d, x, y, z, uw, vel_at, grad);
       // Regularized::stress_from_gradient with the shear rate
       const R kf = -R(2) * (R(1) / R(3)) * rw / p.omega;
       const R Pi[6] = {kf * grad[0][0], kf * grad[1][1], kf * grad[2][2],

@@ -8,6 +8,7 @@
 
 #include "kernels.hpp"
 #include "pair.hpp"
+#include "plane.hpp"
 
 namespace m3lb {
 
@@ -37,7 +38,16 @@ struct KernelSet {
                unsigned nclear, unsigned* host_err, hipStream_t);
   int elem_bytes;    // bytes per stored population
   int real_bytes;    // bytes of the compute type
+  // several steps of a plane box in one launch (plane.hpp); null where not
+  // instantiated (D3Q27, per-node force)
+  void (*plane)(const PlaneArgs&, int shape, int nodes, hipStream_t);
 };
+
+// Regions of the plane kernel (PlaneArgs) and what moves in the box.
+enum PlaneRegion { kPlaneSquare = 0, kPlaneWide = 1 };
+enum PlaneNodes { kPlaneFluid = 0, kPlaneGeom = 1, kPlaneWalls = 2 };
+using PlaneSquare = PlaneShape<32, 32, 1024>;
+using PlaneWide = PlaneShape<64, 32, 512>;
 
 inline unsigned blocks_for(long long n) { return unsigned((n + kBlock - 1) / kBlock); }
 
@@ -144,6 +154,27 @@ struct Launch {
       }
     }
   }
+  static constexpr bool kPlane = K::Q == 9 && !K::FIELD;
+  template <class S>
+  static void plane_s(const PlaneArgs& a, int nodes, hipStream_t s) {
+    const unsigned grid = unsigned(a.ntx) * unsigned(a.nty);
+    if (nodes == kPlaneFluid) k_plane<K, S, false, false><<<grid, S::NT, 0, s>>>(a);
+    else k_plane<K, S, true, false><<<grid, S::NT, 0, s>>>(a);
+  }
+  static void plane(const PlaneArgs& a, int shape, int nodes, hipStream_t s) {
+    if constexpr (kPlane) {
+      if (nodes == kPlaneWalls) {
+        if constexpr (K::OP != M3LB_OP_NULL)
+          k_plane<K, PlaneSquare, true, true>
+              <<<unsigned(a.ntx) * unsigned(a.nty), PlaneSquare::NT, 0, s>>>(a);
+      } else if (shape == kPlaneSquare) {
+        plane_s<PlaneSquare>(a, nodes, s);
+      } else {
+        // 147 KB of LDS with 8-byte populations: one block per CU, slower
+        if constexpr (sizeof(typename K::T) <= 4) plane_s<PlaneWide>(a, nodes, s);
+      }
+    }
+  }
   static void batched(const BatchArgs& a, unsigned grid, hipStream_t s) {
     if constexpr (kBatched) {
       if (a.run == kRunBlockRanges) {
@@ -162,7 +193,8 @@ struct Launch {
                                 snapshot, specular,
                                 kBatched ? batched : nullptr,
                                 kPair ? pair : nullptr,
-                                int(sizeof(typename K::T)), int(sizeof(typename K::R))};
+                                int(sizeof(typename K::T)), int(sizeof(typename K::R)),
+                                kPlane ? plane : nullptr};
     return &t;
   }
 };

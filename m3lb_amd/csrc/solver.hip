@@ -96,6 +96,7 @@ struct Boundaries {
   std::vector<unsigned> don;
   std::vector<double> wtab, wtab0;  // (ux, uy, uz, rho) per state, as the compute type holds them
   bool walls_set = false, has_corners = false, un_on = false;
+  bool local = false;  // straight walls and corners only, and no wall reads another node's set
   int fd_corners = 1;  // fd_corners_ = has_shear_omega<Collision> (FluidSolver.hpp:1287)
   int force_bc = 1;    // force_bc_ (:1288)
   int out_order = 1;   // out_order_ (:1291)
@@ -129,6 +130,11 @@ struct m3lb_solver {
   int device = 0;
   hipStream_t stream = nullptr;
   void* f = nullptr;
+  // second population array of the plane passes (plane.hpp), which read one
+  // array and write the other; alt_synced: the slots that no moving node ever
+  // writes hold the same values in both
+  void* f_alt = nullptr;
+  bool alt_synced = false, alt_failed = false;
   uint64_t stride = 0;  // elements per direction
   uint8_t* flags_d = nullptr;
   std::vector<uint8_t> flags_h;
@@ -432,6 +438,11 @@ int rebuild_plan(m3lb_solver* s) {
   b.nwall = int(walls.size());
   b.nspec = int(spec.size());
   b.nsnap = int(snap_nodes.size());
+  b.local = true;
+  for (size_t w = 0; w < walls.size(); ++w) {
+    b.local = b.local && b.nrm[walls[w]] <= m3lb::kNrmCorner;
+    for (int64_t r : reads[w]) b.local = b.local && r < 0;
+  }
   int rc = upload(b.wlist_d, wlist, s->stream);
   if (!rc) rc = upload(b.slist_d, spec, s->stream);
   if (!rc) rc = upload(b.snap_nodes_d, snap_nodes, s->stream);
@@ -453,9 +464,11 @@ void refresh_geometry(m3lb_solver* s) {
       for (int x = 0; x < d.nx && !geom; ++x)
         geom = s->flags_h[size_t(((z + d.hz) * d.sy + (y + d.hy)) * d.sx + x + d.hx)] != M3LB_FLUID;
   s->geometry = geom;
+  s->alt_synced = false;
 }
 
-m3lb::SeedArgs seed_args(const m3lb_solver* s) {
+m3lb::SeedArgs seed_args(m3lb_solver* s) {
+  s->alt_synced = false;  // a seeding writes slots that no step does
   m3lb::SeedArgs a;
   std::memset(&a, 0, sizeof a);
   a.f = s->f;
@@ -602,6 +615,7 @@ int m3lb_destroy(m3lb_solver* s) {
   if (!s) return M3LB_OK;
   if (s->stream) hipStreamSynchronize(s->stream);
   if (s->f) hipFree(s->f);
+  if (s->f_alt) hipFree(s->f_alt);
   if (s->flags_d) hipFree(s->flags_d);
   if (s->ff_d) hipFree(s->ff_d);
   free_boundaries(s);
@@ -784,6 +798,97 @@ int launch_pair(m3lb_solver* s, const m3lb::StepArgs& a, int parity) {
   return launch_ok();
 }
 
+// Several steps of a plane box per launch (plane.hpp).  Applies to a box whose
+// moving nodes read no other node's set (no outlets, no specular cells, corner
+// stencils on walls) and unless fusion is off.
+struct PlanePlan {
+  int steps = 0;  // most steps per launch, even; 0: one launch per step
+  int shape = 0, nodes = 0;
+};
+
+// Region and steps per launch.  A plane that 32 x 32 regions cover in one
+// round of blocks at 8 steps is bound by launches and by the latency of a
+// step: 8 steps per launch (D2Q9 128^2: FP32 1.28 us per step against 1.5 at
+// 6, 1.8 at 4 and 2.75 one launch per step; FP64 1.40 against 3.0).  Larger
+// ones are bound by traffic and by the work on margins: 4-byte and 2-byte
+// populations take 64 x 32 regions and 6 steps (1024^2 FP32 7.9 us per step,
+// 8.0 at 4 steps, 9.3 with 32 x 32 regions, 11.1 one launch per step; 4096^2
+// 93, 96, 125 and 189), 8-byte ones 32 x 32 and 4 (1024^2 12.0 us, 12.2 at 6,
+// 13.5 with 64 x 32 regions, 23.6 one launch per step; 4096^2 169 and 426).
+PlanePlan plane_plan(const m3lb_solver* s) {
+  PlanePlan p;
+  const Boundaries& b = s->b;
+  const m3lb::Dom& d = s->d;
+  if (!s->ks->plane || s->fusion == M3LB_FUSION_OFF || s->alt_failed || s->Q != 9) return p;
+  if (b.nspec || b.nsnap || (b.nwall && !b.local)) return p;
+  // an unwrapped axis without a halo (one node, not periodic) has no margin
+  if (!(d.px || d.hx) || !(d.py || d.hy)) return p;
+  p.nodes = b.nwall ? m3lb::kPlaneWalls
+                    : (s->geometry || d.hx || d.hy ? m3lb::kPlaneGeom : m3lb::kPlaneFluid);
+  const int core8 = m3lb::PlaneSquare::RX - 2 * (b.nwall ? 10 : 8);
+  const int64_t blocks8 = int64_t((d.sx + core8 - 1) / core8) * ((d.sy + core8 - 1) / core8);
+  p.shape = m3lb::kPlaneSquare;
+  if (blocks8 <= (b.nwall ? 1 : 2) * int64_t(s->cus)) {
+    p.steps = 8;
+  } else if (b.nwall || s->ks->elem_bytes == 8) {
+    p.steps = 4;
+  } else {
+    p.shape = m3lb::kPlaneWide;
+    p.steps = 6;
+    // 2-byte populations beyond the caches' reach of one XCD gain little (D2Q9
+    // CM 2048^2, us per step: FP16 27.2 against 27.3, BF16 25.7 / 28.1, I16
+    // 24.7 / 28.5), and E2M13 (32.0 / 30.6, its codec runs on the margins too)
+    // and boxes with geometry (FP16 28.2 / 27.6, E2M13 34.0 / 29.4) lose
+    const uint64_t bytes = s->stride * uint64_t(s->Q) * uint64_t(s->ks->elem_bytes);
+    if (s->ks->elem_bytes == 2 && bytes > (32u << 20) &&
+        (s->cfg.dtype == M3LB_E2M13 || p.nodes == m3lb::kPlaneGeom))
+      p.steps = 0;
+  }
+  return p;
+}
+
+// The second population array: allocated at the first pass, and given the
+// slots no moving node writes whenever those may have changed.  A failed
+// allocation leaves the box to one launch per step.
+int ensure_alt(m3lb_solver* s, bool statics) {
+  const size_t bytes = size_t(s->stride) * size_t(s->Q) * size_t(s->ks->elem_bytes);
+  if (!s->f_alt) {
+    if (hipMalloc(&s->f_alt, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      s->f_alt = nullptr;
+      s->alt_failed = true;
+      return M3LB_OK;
+    }
+    s->alt_synced = false;
+  }
+  if (statics && !s->alt_synced)
+    HIP_OK(hipMemcpyAsync(s->f_alt, s->f, bytes, hipMemcpyDeviceToDevice, s->stream));
+  s->alt_synced = true;
+  return M3LB_OK;
+}
+
+// `steps` (even) steps from an even one.
+int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& wa,
+                 const PlanePlan& p, int steps) {
+  m3lb::PlaneArgs pa;
+  std::memset(&pa, 0, sizeof pa);
+  pa.a = a;
+  pa.a.remap = 8;
+  for (int j = 0; j < 4; ++j) pa.a.macro[j] = nullptr;
+  pa.w = wa;
+  pa.out = s->f_alt;
+  pa.steps = steps;
+  pa.margin = steps + (p.nodes == m3lb::kPlaneWalls ? 2 : 0);
+  const bool wide = p.shape == m3lb::kPlaneWide;
+  const int cx = (wide ? m3lb::PlaneWide::RX : m3lb::PlaneSquare::RX) - 2 * pa.margin;
+  const int cy = (wide ? m3lb::PlaneWide::RY : m3lb::PlaneSquare::RY) - 2 * pa.margin;
+  pa.ntx = (s->d.sx + cx - 1) / cx;
+  pa.nty = (s->d.sy + cy - 1) / cy;
+  s->ks->plane(pa, p.shape, p.nodes, s->stream);
+  std::swap(s->f, s->f_alt);
+  return launch_ok();
+}
+
 }  // namespace
 
 extern "C" {
@@ -849,8 +954,27 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   na.out = b.snap_d;
   for (int q = 0; q < 27; ++q) na.inv_scale[q] = s->inv_scale[q];
   const bool pairs = pair_eligible(s, a);
+  PlanePlan plane = plane_plan(s);
+  if (plane.steps && nsteps - int(s->t % 2) - (store_macroscopic ? 1 : 0) >= 2) {
+    const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid);
+    if (rc) return rc;
+    if (s->alt_failed) plane.steps = 0;
+  }
   for (int k = 0; k < nsteps; ++k) {
     const bool last = k == nsteps - 1;
+    // the plane passes: even numbers of steps from an even one (never the
+    // step that stores the macroscopic fields)
+    const int left = nsteps - k - (store_macroscopic ? 1 : 0);
+    if (plane.steps && left >= 2 && s->t % 2 == 0) {
+      const int n = std::min(plane.steps, left & ~1);
+      const int rc = launch_plane(s, a, wa, plane, n);
+      if (rc) return rc;
+      a.f = wa.f = sa.f = s->f;
+      na.f = s->f;
+      s->t += uint64_t(n);
+      k += n - 1;
+      continue;
+    }
     // two steps in one pass while two are left (never the step that stores
     // the macroscopic fields)
     if (pairs && k + 1 < nsteps && !(store_macroscopic && k + 2 == nsteps)) {
@@ -1626,6 +1750,7 @@ static int apply_scales(m3lb_solver* s, const double* want) {
   for (int q = 0; q < 27; ++q) r.r[q] = 1.0f;
   for (int q = 0; q < s->Q; ++q) r.r[q] = float(want[q] / double(s->scale[q]));
   const unsigned grid = reduce_grid(s);
+  s->alt_synced = false;
   s->ks->rescale(s->f, s->stride, s->d.np, r, grid, s->stream);
   int rc = launch_ok();
   if (rc) return rc;
@@ -1684,6 +1809,7 @@ int m3lb_device_bytes(const m3lb_solver* s, uint64_t* bytes) {
   for (void* p : s->macro_d)
     if (p) b += uint64_t(s->d.np) * uint64_t(s->ks->real_bytes);
   b += s->partial_n * sizeof(double);
+  if (s->f_alt) b += s->stride * uint64_t(s->Q) * uint64_t(s->ks->elem_bytes);
   *bytes = b;
   return M3LB_OK;
 }
