@@ -521,10 +521,21 @@ struct SeedArgs {
   int parity;
   int mode;
   double rho0, u0[3];
-  const double* field[4];  // rho, ux, uy, uz (padded), kSeedField
-  const double* arr;       // (n, q) logical populations, kSeedArray
+  const void* field[4];  // rho, ux, uy, uz (padded, compute type), kSeedField
+  const void* arr;       // (n, q) logical populations (compute type), kSeedArray
   float scale[27];
 };
+
+__device__ __forceinline__ int shift_axis(int v, int h, int n, int s, int per) {
+  if (per) {
+    if (v < h) return v + n;
+    if (v >= h + n) return v - n;
+    return v;
+  }
+  if (v < 0) return 0;
+  if (v >= s) return s - 1;
+  return v;
+}
 
 // Along one axis: the largest coordinate v with shift(v + e) == m, or -1.
 __device__ __forceinline__ int writer_axis(int m, int e, int n, int s, int per) {
@@ -575,8 +586,8 @@ __device__ __forceinline__ void seed_value_of(const SeedArgs& a, int n, typename
       seed<K>(v, R(1), R(0), R(0), R(0));
     }
   } else {
-    if (fluid)
-      seed<K>(v, R(a.field[0][n]), R(a.field[1][n]), R(a.field[2][n]), R(a.field[3][n]));
+    auto at = [&](int k) { return static_cast<const R*>(a.field[k])[n]; };
+    if (fluid) seed<K>(v, at(0), at(1), at(2), at(3));
     else seed<K>(v, R(1), R(0), R(0), R(0));
   }
 }
@@ -626,7 +637,7 @@ __global__ void __launch_bounds__(kBlock) k_seed(SeedArgs a) {
     if (w < 0) return;  // no node writes this slot: it keeps its value
     R val;
     if (a.mode == kSeedArray) {
-      val = R(a.arr[uint64_t(w) * Q + i]);
+      val = static_cast<const R*>(a.arr)[uint64_t(w) * Q + i];
     } else if (w == m) {
       val = R(0);
       sfor<Q>([&](auto J) { if (int(J) == i) val = own[int(J)]; });
@@ -651,8 +662,10 @@ struct ReadArgs {
   const uint8_t* flags;
   Dom d;
   int parity;
-  double* out;       // gather: (n, q); macro: rho, ux, uy, uz planes
-  double* out2[4];
+  void* out;         // gather: (n, q), compute type; reductions: FP64 partials
+  void* out2[4];     // macro: rho, ux, uy, uz, compute type, from node n0 on
+  int n0, n1;        // macro, gather, storage: the padded nodes [n0, n1)
+  FastDiv div_sx, div_sy;  // padded node index -> coordinates
   float inv_scale[27];
   double omega, omega_m, omega_b, F[3];
   const void* ff;  // per-node force planes (FIELD only)
@@ -670,15 +683,12 @@ struct ReadArgs {
   const uint8_t* spec_faces;  // on-node specular face masks, or null
 };
 
-__device__ __forceinline__ int shift_axis(int v, int h, int n, int s, int per) {
-  if (per) {
-    if (v < h) return v + n;
-    if (v >= h + n) return v - n;
-    return v;
-  }
-  if (v < 0) return 0;
-  if (v >= s) return s - 1;
-  return v;
+// Padded coordinates of padded node n.
+__device__ __forceinline__ void padded_coords(const ReadArgs& a, int n, int& x, int& y, int& z) {
+  const unsigned row = fd_div(a.div_sx, unsigned(n));
+  z = int(fd_div(a.div_sy, row));
+  x = n - int(row) * a.d.sx;
+  y = int(row) - z * a.d.sy;
 }
 
 // Stored value of the population travelling in direction i that arrives at
@@ -706,17 +716,30 @@ __device__ __forceinline__ typename K::R arriving(const ReadArgs& a, int n, int 
   return C::dec(A[uint64_t(slot) * a.stride + unsigned(node)], a.inv_scale[slot]);
 }
 
+// Writes the block's (node, direction) values in address order: the Q values
+// of a node are consecutive, so stored from the registers every store of a
+// wave would touch 64 rows of the output; through LDS (the row length Q is
+// odd, so no bank conflicts) they are contiguous, which the output's place,
+// pinned host memory, needs.
+template <class K, class Value>
+__device__ __forceinline__ void write_rows(const ReadArgs& a, int n, Value&& value) {
+  using R = typename K::R;
+  constexpr int Q = K::Q;
+  __shared__ R rows[kBlock * Q];
+  if (n < a.n1) sfor<Q>([&](auto I) { rows[int(threadIdx.x) * Q + int(I)] = value(I); });
+  __syncthreads();
+  const int first = a.n0 + int(blockIdx.x) * kBlock;
+  const int count = (a.n1 - first < kBlock ? a.n1 - first : kBlock) * Q;
+  R* out = static_cast<R*>(a.out) + size_t(first - a.n0) * Q;
+  for (int k = int(threadIdx.x); k < count; k += kBlock) out[k] = rows[k];
+}
+
 template <class K>
 __global__ void __launch_bounds__(kBlock) k_gather(ReadArgs a) {
-  constexpr int Q = K::Q;
-  const int n = blockIdx.x * kBlock + threadIdx.x;
-  const Dom& d = a.d;
-  if (n >= d.np) return;
-  const int x = n % d.sx, y = (n / d.sx) % d.sy, z = n / (d.sx * d.sy);
-  sfor<Q>([&](auto I) {
-    constexpr int i = I;
-    a.out[uint64_t(n) * Q + i] = double(arriving<K, i>(a, n, x, y, z));
-  });
+  const int n = a.n0 + int(blockIdx.x) * kBlock + int(threadIdx.x);
+  int x, y, z;
+  padded_coords(a, n, x, y, z);
+  write_rows<K>(a, n, [&](auto I) { return arriving<K, int(I)>(a, n, x, y, z); });
 }
 
 // Raw slot image (EsotericPull::storage()), (n, q) ordered.
@@ -724,14 +747,11 @@ template <class K>
 __global__ void __launch_bounds__(kBlock) k_storage(ReadArgs a) {
   using T = typename K::T;
   using C = typename K::C;
-  constexpr int Q = K::Q;
-  const int n = blockIdx.x * kBlock + threadIdx.x;
-  if (n >= a.d.np) return;
+  const int n = a.n0 + int(blockIdx.x) * kBlock + int(threadIdx.x);
   const T* A = static_cast<const T*>(a.f);
-  sfor<Q>([&](auto I) {
+  write_rows<K>(a, n, [&](auto I) {
     constexpr int q = I;
-    a.out[uint64_t(n) * Q + q] = double(C::dec(A[uint64_t(q) * a.stride + unsigned(n)],
-                                               a.inv_scale[q]));
+    return C::dec(A[uint64_t(q) * a.stride + unsigned(n)], a.inv_scale[q]);
   });
 }
 
@@ -752,14 +772,14 @@ template <class K>
 __global__ void __launch_bounds__(kBlock) k_macro(ReadArgs a) {
   using R = typename K::R;
   using T = typename K::T;
-  const int n = blockIdx.x * kBlock + threadIdx.x;
+  const int n = a.n0 + int(blockIdx.x) * kBlock + int(threadIdx.x);
   const Dom& d = a.d;
-  if (n >= d.np) return;
+  if (n >= a.n1) return;
   double r = 0, ux = 0, uy = 0, uz = 0;
   if (a.flags[n] == M3LB_FLUID) {
     int x, y, z;
-    interior_coords<K, 0>(d, n, x, y, z);
-    const Offs o = offsets(d, x, y, z);
+    padded_coords(a, n, x, y, z);
+    const Offs o = offsets(d, x - d.hx, y - d.hy, z - d.hz);
     Params<R> p;
     p.omega = R(a.omega); p.omega_m = R(a.omega_m); p.omega_b = R(a.omega_b);
     p.F[0] = R(a.F[0]); p.F[1] = R(a.F[1]); p.F[2] = R(a.F[2]);
@@ -776,8 +796,8 @@ __global__ void __launch_bounds__(kBlock) k_macro(ReadArgs a) {
     // macro_kernel's SpecNode path (FluidSolver.hpp:1057-1077): raw moments
     // of the mirrored incoming set
     int x, y, z;
-    interior_coords<K, 0>(d, n, x, y, z);
-    const Offs o = offsets(d, x, y, z);
+    padded_coords(a, n, x, y, z);
+    const Offs o = offsets(d, x - d.hx, y - d.hy, z - d.hz);
     R f[K::Q];
     const T* A = static_cast<const T*>(a.f);
     if (a.parity == 0) load_node<K, 0>(A, a.stride, unsigned(n), o, a.inv_scale, f);
@@ -795,10 +815,9 @@ __global__ void __launch_bounds__(kBlock) k_macro(ReadArgs a) {
     const R ir = R(1) / sm;
     r = double(sm); ux = double(mx * ir); uy = double(my * ir); uz = double(mz * ir);
   }
-  if (a.out2[0]) a.out2[0][n] = r;
-  if (a.out2[1]) a.out2[1][n] = ux;
-  if (a.out2[2]) a.out2[2][n] = uy;
-  if (a.out2[3]) a.out2[3][n] = uz;
+  const double v[4] = {r, ux, uy, uz};  // compute-type values: stored exactly
+  for (int k = 0; k < 4; ++k)
+    if (a.out2[k]) static_cast<R*>(a.out2[k])[n - a.n0] = R(v[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -842,8 +861,8 @@ __global__ void __launch_bounds__(kBlock) k_reduce_mass(ReadArgs a) {
   for (int n = blockIdx.x * kBlock + threadIdx.x; n < d.np; n += gridDim.x * kBlock) {
     if (!fluid_like(a.flags[n])) continue;
     int x, y, z;
-    interior_coords<K, 0>(d, n, x, y, z);
-    const Offs o = offsets(d, x, y, z);
+    padded_coords(a, n, x, y, z);
+    const Offs o = offsets(d, x - d.hx, y - d.hy, z - d.hz);
     Params<R> p;
     p.omega = R(a.omega); p.omega_m = R(a.omega_m); p.omega_b = R(a.omega_b);
     p.F[0] = R(a.F[0]); p.F[1] = R(a.F[1]); p.F[2] = R(a.F[2]);
@@ -861,7 +880,7 @@ __global__ void __launch_bounds__(kBlock) k_reduce_mass(ReadArgs a) {
     acc[2] += double(r * m.uy);
     acc[3] += double(r * m.uz);
   }
-  block_sum<4>(acc, a.out);
+  block_sum<4>(acc, static_cast<double*>(a.out));
 }
 
 // Momentum exchange with a body (validation/square_cylinder.cpp:27-50,
@@ -1458,22 +1477,30 @@ __device__ void wall_macro(const ReadArgs& a, unsigned n, double& r, double& ux,
   ux = double(uw[0]); uy = double(uw[1]); uz = double(uw[2]);
 }
 
+// body: interior mask (x fastest), nonzero = in the body; null: every Solid node.
 template <class K>
 __global__ void __launch_bounds__(kBlock) k_momentum_exchange(ReadArgs a, const uint8_t* body) {
   using R = typename K::R;
   constexpr int Q = K::Q;
   const Dom& d = a.d;
+  auto in_body = [&](int mx, int my, int mz) -> bool {
+    if (!body) return a.flags[(mz * d.sy + my) * d.sx + mx] == M3LB_SOLID;
+    const int x = mx - d.hx, y = my - d.hy, z = mz - d.hz;
+    return unsigned(x) < unsigned(d.nx) && unsigned(y) < unsigned(d.ny) &&
+           unsigned(z) < unsigned(d.nz) && body[(size_t(z) * d.ny + y) * d.nx + x] != 0;
+  };
   double acc[3] = {0, 0, 0};
   for (int n = blockIdx.x * kBlock + threadIdx.x; n < d.np; n += gridDim.x * kBlock) {
     if (a.flags[n] != M3LB_FLUID) continue;
-    const int x = n % d.sx, y = (n / d.sx) % d.sy, z = n / (d.sx * d.sy);
+    int x, y, z;
+    padded_coords(a, n, x, y, z);
     sfor<Q - 1>([&](auto I) {
       constexpr int i = int(I) + 1;
       constexpr int io = opp<Q>(i);
       const int mx = shift_axis(x + Lat<Q>::cx[i], d.hx, d.nx, d.sx, d.px);
       const int my = shift_axis(y + Lat<Q>::cy[i], d.hy, d.ny, d.sy, d.py);
       const int mz = shift_axis(z + Lat<Q>::cz[i], d.hz, d.nz, d.sz, d.pz);
-      if (!body[(mz * d.sy + my) * d.sx + mx]) return;
+      if (!in_body(mx, my, mz)) return;
       R f = arriving<K, io>(a, n, x, y, z);
       if constexpr (K::SHIFTED) f = f + weight<K>(io);
       const double fd = double(f);
@@ -1482,7 +1509,7 @@ __global__ void __launch_bounds__(kBlock) k_momentum_exchange(ReadArgs a, const 
       acc[2] += 2.0 * Lat<Q>::cz[i] * fd;
     });
   }
-  block_sum<3>(acc, a.out);
+  block_sum<3>(acc, static_cast<double*>(a.out));
 }
 
 // Exact sum of every slot: value * 2^100 truncated toward zero, summed as a
@@ -1586,7 +1613,7 @@ __global__ void __launch_bounds__(kBlock) k_absmax(ReadArgs a) {
     if (threadIdx.x == 0) {
       double m = 0;
       for (int k = 0; k < kBlock; ++k) m = lds[k] > m ? lds[k] : m;
-      a.out[uint64_t(blockIdx.x) * Q + q] = m;
+      static_cast<double*>(a.out)[uint64_t(blockIdx.x) * Q + q] = m;
     }
     __syncthreads();
   });

@@ -84,13 +84,13 @@ struct Launch {
     k_seed<K><<<blocks_for(a.d.np), kBlock, 0, s>>>(a);
   }
   static void gather(const ReadArgs& a, hipStream_t s) {
-    k_gather<K><<<blocks_for(a.d.np), kBlock, 0, s>>>(a);
+    k_gather<K><<<blocks_for((long long)(a.n1) - a.n0), kBlock, 0, s>>>(a);
   }
   static void storage(const ReadArgs& a, hipStream_t s) {
-    k_storage<K><<<blocks_for(a.d.np), kBlock, 0, s>>>(a);
+    k_storage<K><<<blocks_for((long long)(a.n1) - a.n0), kBlock, 0, s>>>(a);
   }
   static void macro(const ReadArgs& a, hipStream_t s) {
-    k_macro<K><<<blocks_for(a.d.np), kBlock, 0, s>>>(a);
+    k_macro<K><<<blocks_for((long long)(a.n1) - a.n0), kBlock, 0, s>>>(a);
   }
   static void reduce_mass(const ReadArgs& a, unsigned grid, hipStream_t s) {
     k_reduce_mass<K><<<grid, kBlock, 0, s>>>(a);

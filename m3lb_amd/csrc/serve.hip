@@ -25,6 +25,7 @@
 #include "launch.hpp"
 #include "serve_plan.hpp"
 #include "scales.hpp"
+#include "transfer.hpp"
 
 using m3lb::BoxDesc;
 using m3lb::KernelSet;
@@ -258,6 +259,10 @@ m3lb::ReadArgs read_args(const m3lb_server* s, const Box& b, double* out) {
   a.stride = b.stride;
   a.flags = b.desc.flags;
   a.d = b.d;
+  a.div_sx = m3lb::make_fastdiv(uint32_t(b.d.sx));
+  a.div_sy = m3lb::make_fastdiv(uint32_t(b.d.sy));
+  a.n0 = 0;
+  a.n1 = b.d.np;
   a.parity = b.parity;
   a.out = out;
   a.omega = b.req.omega;
@@ -658,6 +663,7 @@ int m3lb_srv_destroy(m3lb_server* s) {
   if (s->summary_h) (void)hipHostFree(s->summary_h);
   if (s->arena_d) (void)hipFree(s->arena_d);
   if (s->stream) (void)hipStreamDestroy(s->stream);
+  m3lb::staging_release();
   delete s;
   return M3LB_OK;
 }
@@ -670,6 +676,7 @@ int m3lb_srv_create(const m3lb_server_config* cfg, m3lb_server** out) {
   const KernelSet* ks = m3lb::kernel_set(cfg->lattice, cfg->op, cfg->storage, cfg->dtype, cfg->forcing);
   if (!ks || !ks->batched) return err(M3LB_EINVAL, "no batched kernel for this configuration");
   m3lb_server* s = new m3lb_server();
+  m3lb::staging_acquire();
   s->cfg = *cfg;
   s->ks = ks;
   s->Q = cfg->lattice;
@@ -835,22 +842,8 @@ int m3lb_srv_fetch_macroscopic(m3lb_server* s, int64_t id, double* rho, double* 
   Box* b;
   int rc = kept_done(s, id, &b);
   if (rc) return rc;
-  const size_t np = size_t(b->d.np);
-  double* buf = nullptr;
-  SRV_HIP(hipMalloc(&buf, 4 * np * sizeof(double)));
-  m3lb::ReadArgs a = read_args(s, *b, nullptr);
-  for (int k = 0; k < 4; ++k) a.out2[k] = buf + k * np;
-  s->ks->macro(a, s->stream);
-  rc = launch_ok();
-  double* dst[4] = {rho, ux, uy, uz};
-  for (int k = 0; k < 4 && !rc; ++k)
-    if (dst[k] && hipMemcpyAsync(dst[k], buf + k * np, np * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-      rc = err(M3LB_EDEVICE, "macroscopic download failed");
-  const hipError_t e = hipStreamSynchronize(s->stream);
-  (void)hipFree(buf);
-  if (rc) return rc;
-  if (e != hipSuccess) return err(M3LB_EDEVICE, hipGetErrorString(e));
-  return M3LB_OK;
+  double* const dst[4] = {rho, ux, uy, uz};
+  return m3lb::read_macroscopic(s->ks, read_args(s, *b, nullptr), s->device, s->stream, dst);
 }
 
 int m3lb_srv_fetch_populations(m3lb_server* s, int64_t id, double* out) {
@@ -858,18 +851,7 @@ int m3lb_srv_fetch_populations(m3lb_server* s, int64_t id, double* out) {
   Box* b;
   int rc = kept_done(s, id, &b);
   if (rc) return rc;
-  const size_t n = size_t(b->d.np) * size_t(s->Q);
-  double* buf = nullptr;
-  SRV_HIP(hipMalloc(&buf, n * sizeof(double)));
-  s->ks->gather(read_args(s, *b, buf), s->stream);
-  rc = launch_ok();
-  if (!rc && hipMemcpyAsync(out, buf, n * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-    rc = err(M3LB_EDEVICE, "population download failed");
-  const hipError_t e = hipStreamSynchronize(s->stream);
-  (void)hipFree(buf);
-  if (rc) return rc;
-  if (e != hipSuccess) return err(M3LB_EDEVICE, hipGetErrorString(e));
-  return M3LB_OK;
+  return m3lb::read_populations(s->ks, read_args(s, *b, nullptr), s->Q, true, s->device, s->stream, out);
 }
 
 int m3lb_srv_release(m3lb_server* s, int64_t id) {

@@ -14,6 +14,7 @@
 
 #include "launch.hpp"
 #include "scales.hpp"
+#include "transfer.hpp"
 
 using m3lb::KernelSet;
 
@@ -143,6 +144,8 @@ struct m3lb_solver {
   bool macro_valid = false;
   double* partial_d = nullptr;  // per-block partials
   size_t partial_n = 0;
+  void* work_d = nullptr;  // scratch of the readouts and uploads, kept up to kKeptWork bytes
+  size_t work_n = 0;
   uint64_t t = 0;
   float scale[27];
   float inv_scale[27];
@@ -195,6 +198,25 @@ int ensure_partials(m3lb_solver* s, size_t n_doubles) {
   return M3LB_OK;
 }
 
+// Scratch of at least `bytes` for one call; drop_work after it gives a large
+// one back.
+constexpr size_t kKeptWork = 64u << 20;
+int ensure_work(m3lb_solver* s, size_t bytes) {
+  if (s->work_n >= bytes) return M3LB_OK;
+  if (s->work_d) HIP_OK(hipFree(s->work_d));
+  s->work_d = nullptr;
+  s->work_n = 0;
+  HIP_OK(hipMalloc(&s->work_d, bytes));
+  s->work_n = bytes;
+  return M3LB_OK;
+}
+void drop_work(m3lb_solver* s) {
+  if (s->work_n <= kKeptWork) return;
+  (void)hipFree(s->work_d);
+  s->work_d = nullptr;
+  s->work_n = 0;
+}
+
 m3lb::StepArgs step_args(const m3lb_solver* s) {
   m3lb::StepArgs a;
   std::memset(&a, 0, sizeof a);
@@ -228,6 +250,10 @@ m3lb::ReadArgs read_args(const m3lb_solver* s) {
   a.stride = s->stride;
   a.flags = s->flags_d;
   a.d = s->d;
+  a.div_sx = m3lb::make_fastdiv(uint32_t(s->d.sx));
+  a.div_sy = m3lb::make_fastdiv(uint32_t(s->d.sy));
+  a.n0 = 0;
+  a.n1 = s->d.np;
   a.parity = int(s->t % 2);
   a.omega = s->cfg.omega;
   a.omega_m = s->cfg.omega_minus;
@@ -540,6 +566,7 @@ int m3lb_create(const m3lb_config* cfg, m3lb_solver** out) {
     return fail(M3LB_EINVAL, "one direction of the population array exceeds 4 GiB");
 
   m3lb_solver* s = new m3lb_solver();
+  m3lb::staging_acquire();
   s->cfg = *cfg;
   s->Q = cfg->lattice;
   std::memcpy(s->dom, dom, sizeof dom);
@@ -622,11 +649,13 @@ int m3lb_destroy(m3lb_solver* s) {
   for (void* p : s->macro_d)
     if (p) hipFree(p);
   if (s->partial_d) hipFree(s->partial_d);
+  if (s->work_d) hipFree(s->work_d);
   if (s->pair_sync) hipFree(s->pair_sync);
   if (s->pair_err_h) hipHostFree(s->pair_err_h);
   if (s->ev0) hipEventDestroy(s->ev0);
   if (s->ev1) hipEventDestroy(s->ev1);
   if (s->stream) hipStreamDestroy(s->stream);
+  m3lb::staging_release();
   delete s;
   return M3LB_OK;
 }
@@ -681,38 +710,39 @@ int m3lb_initialize_field(m3lb_solver* s, const double* rho, const double* ux, c
   s->t = 0;
   s->macro_valid = false;
   provisional_scales(s);
-  const size_t np = size_t(s->d.np);
-  double* buf = nullptr;
-  HIP_OK(hipMalloc(&buf, 4 * np * sizeof(double)));
+  const size_t np = size_t(s->d.np), rb = size_t(s->ks->real_bytes);
+  int rc = ensure_work(s, 4 * np * rb);
+  if (rc) return rc;
+  char* buf = static_cast<char*>(s->work_d);
   const double* src[4] = {rho, ux, uy, uz};
-  for (int k = 0; k < 4; ++k)
-    HIP_OK(hipMemcpyAsync(buf + k * np, src[k], np * sizeof(double), hipMemcpyHostToDevice, s->stream));
   m3lb::SeedArgs a = seed_args(s);
   a.mode = m3lb::kSeedField;
-  for (int k = 0; k < 4; ++k) a.field[k] = buf + k * np;
-  const int rc = seed_calibrated(s, a);  // synchronises before returning
-  (void)hipFree(buf);
+  for (int k = 0; k < 4 && !rc; ++k) {
+    a.field[k] = buf + size_t(k) * np * rb;
+    rc = m3lb::upload_real(buf + size_t(k) * np * rb, src[k], np, int(rb), s->device, s->stream);
+  }
+  if (!rc) rc = seed_calibrated(s, a);  // synchronises before returning
+  drop_work(s);
   return rc;
 }
 
 int m3lb_seed_populations(m3lb_solver* s, const double* in) {
   if (!s || !in) return fail(M3LB_EINVAL, "null argument");
   s->macro_valid = false;
-  const size_t n = size_t(s->d.np) * size_t(s->Q);
-  double* buf = nullptr;
-  HIP_OK(hipMalloc(&buf, n * sizeof(double)));
-  HIP_OK(hipMemcpyAsync(buf, in, n * sizeof(double), hipMemcpyHostToDevice, s->stream));
-  m3lb::SeedArgs a = seed_args(s);
-  a.mode = m3lb::kSeedArray;
-  a.arr = buf;
-  s->ks->seed(a, s->stream);
-  int rc = launch_ok();
-  hipError_t e = hipStreamSynchronize(s->stream);
-  hipFree(buf);
-  if (rc) return rc;
-  if (e != hipSuccess) return fail(M3LB_EDEVICE, hipGetErrorString(e));
-  SYNC_OK(s);  // reports a failed two-step pass
-  return M3LB_OK;
+  const size_t n = size_t(s->d.np) * size_t(s->Q), rb = size_t(s->ks->real_bytes);
+  int rc = ensure_work(s, n * rb);
+  if (!rc) rc = m3lb::upload_real(s->work_d, in, n, int(rb), s->device, s->stream);
+  if (!rc) {
+    m3lb::SeedArgs a = seed_args(s);
+    a.mode = m3lb::kSeedArray;
+    a.arr = s->work_d;
+    s->ks->seed(a, s->stream);
+    rc = launch_ok();
+    const int sync_rc = stream_sync(s);  // reports a failed two-step pass
+    if (!rc) rc = sync_rc;
+  }
+  drop_work(s);
+  return rc;
 }
 
 }  // extern "C"
@@ -1033,21 +1063,9 @@ int m3lb_time_steps(m3lb_solver* s, int32_t nsteps, double* ms) {
 
 int m3lb_compute_macroscopic(m3lb_solver* s, double* rho, double* ux, double* uy, double* uz) {
   if (!s) return fail(M3LB_EINVAL, "null handle");
-  const size_t np = size_t(s->d.np);
-  double* buf = nullptr;
-  HIP_OK(hipMalloc(&buf, 4 * np * sizeof(double)));
-  m3lb::ReadArgs a = read_args(s);
-  for (int k = 0; k < 4; ++k) a.out2[k] = buf + k * np;
-  s->ks->macro(a, s->stream);
-  int rc = launch_ok();
-  double* dst[4] = {rho, ux, uy, uz};
-  for (int k = 0; k < 4 && !rc; ++k)
-    if (dst[k] && hipMemcpyAsync(dst[k], buf + k * np, np * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-      rc = fail(M3LB_EDEVICE, "macroscopic download failed");
-  hipError_t e = hipStreamSynchronize(s->stream);
-  hipFree(buf);
+  double* const dst[4] = {rho, ux, uy, uz};
+  const int rc = m3lb::read_macroscopic(s->ks, read_args(s), s->device, s->stream, dst);
   if (rc) return rc;
-  if (e != hipSuccess) return fail(M3LB_EDEVICE, hipGetErrorString(e));
   SYNC_OK(s);  // reports a failed two-step pass
   return M3LB_OK;
 }
@@ -1088,12 +1106,9 @@ static int reduce4(m3lb_solver* s, double out[4]) {
   s->ks->reduce_mass(a, grid, s->stream);
   rc = launch_ok();
   if (rc) return rc;
-  std::vector<double> h(size_t(grid) * 4);
-  HIP_OK(hipMemcpyAsync(h.data(), s->partial_d, h.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+  rc = m3lb::read_column_sums(s->partial_d, grid, 4, s->device, s->stream, out);
+  if (rc) return rc;
   SYNC_OK(s);
-  for (int k = 0; k < 4; ++k) out[k] = 0;
-  for (unsigned b = 0; b < grid; ++b)
-    for (int k = 0; k < 4; ++k) out[k] += h[size_t(b) * 4 + k];
   return M3LB_OK;
 }
 
@@ -1192,43 +1207,26 @@ int m3lb_total_momentum(m3lb_solver* s, int32_t axis, double* out) {
 
 int m3lb_momentum_exchange(m3lb_solver* s, const uint8_t* body, double force[3]) {
   if (!s || !force) return fail(M3LB_EINVAL, "null argument");
-  const m3lb::Dom& d = s->d;
-  std::vector<uint8_t> pad(size_t(d.np), 0);
-  if (body) {
-    size_t k = 0;
-    for (int z = 0; z < d.nz; ++z)
-      for (int y = 0; y < d.ny; ++y)
-        for (int x = 0; x < d.nx; ++x, ++k)
-          pad[size_t(((z + d.hz) * d.sy + (y + d.hy)) * d.sx + x + d.hx)] = body[k] ? 1 : 0;
-  } else {
-    for (size_t n = 0; n < pad.size(); ++n) pad[n] = s->flags_h[n] == M3LB_SOLID ? 1 : 0;
-  }
   const unsigned grid = reduce_grid(s);
   int rc = ensure_partials(s, size_t(grid) * 3);
   if (rc) return rc;
-  uint8_t* body_d = nullptr;
-  HIP_OK(hipMalloc(&body_d, pad.size()));
-  rc = M3LB_OK;
-  if (hipMemcpyAsync(body_d, pad.data(), pad.size(), hipMemcpyHostToDevice, s->stream) != hipSuccess)
-    rc = fail(M3LB_EDEVICE, "body upload failed");
-  std::vector<double> h(size_t(grid) * 3);
+  const uint8_t* body_d = nullptr;
+  if (body) {
+    const size_t ni = size_t(s->d.nx) * size_t(s->d.ny) * size_t(s->d.nz);
+    rc = ensure_work(s, ni);
+    if (!rc) rc = m3lb::upload_bytes(s->work_d, body, ni, s->device, s->stream);
+    body_d = static_cast<const uint8_t*>(s->work_d);
+  }
   if (!rc) {
     m3lb::ReadArgs a = read_args(s);
     a.out = s->partial_d;
     s->ks->exchange(a, body_d, grid, s->stream);
     rc = launch_ok();
   }
-  if (!rc && hipMemcpyAsync(h.data(), s->partial_d, h.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-    rc = fail(M3LB_EDEVICE, "partials download failed");
-  const hipError_t e = hipStreamSynchronize(s->stream);
-  (void)hipFree(body_d);
-  if (rc) return rc;
-  if (e != hipSuccess) return fail(M3LB_EDEVICE, hipGetErrorString(e));
-  SYNC_OK(s);  // reports a failed two-step pass
-  for (int k = 0; k < 3; ++k) force[k] = 0;
-  for (unsigned b = 0; b < grid; ++b)
-    for (int k = 0; k < 3; ++k) force[k] += h[size_t(b) * 3 + k];
-  return M3LB_OK;
+  if (!rc) rc = m3lb::read_column_sums(s->partial_d, grid, 3, s->device, s->stream, force);
+  const int sync_rc = stream_sync(s);  // reports a failed two-step pass
+  drop_work(s);
+  return rc ? rc : sync_rc;
 }
 
 int m3lb_storage_sum_exact(m3lb_solver* s, int64_t out[2]) {
@@ -1257,36 +1255,47 @@ int m3lb_storage_sum_exact(m3lb_solver* s, int64_t out[2]) {
 // E = sum 1/2|u|^2 and Omega = sum 1/2|curl u|^2 over interior nodes with
 // periodic-wrap central differences (validation/Campaign.hpp:99-130).
 namespace {
-__global__ void __launch_bounds__(m3lb::kBlock) k_energy(m3lb::Dom d, const double* ux,
-                                                         const double* uy, const double* uz,
-                                                         double* out, int* finite) {
-  const long long N = (long long)d.nx * d.ny * d.nz;
-  double acc[2] = {0, 0};
-  bool ok = true;
-  for (long long i = blockIdx.x * (long long)m3lb::kBlock + threadIdx.x; i < N;
-       i += (long long)gridDim.x * m3lb::kBlock) {
-    const int x = int(i % d.nx), y = int((i / d.nx) % d.ny), z = int(i / ((long long)d.nx * d.ny));
-    auto id = [&](int xx, int yy, int zz) {
-      xx = (xx + d.nx) % d.nx; yy = (yy + d.ny) % d.ny; zz = (zz + d.nz) % d.nz;
-      return ((zz + d.hz) * d.sy + (yy + d.hy)) * d.sx + xx + d.hx;
+constexpr int kWholeBox = -2;
+// u holds the three velocity components, `comp` values apart, of whole padded
+// planes: of the box (zfirst = kWholeBox), or from interior plane zfirst on.  Sums over
+// the interior planes [z0, z1); the third column counts non-finite nodes.
+template <class R>
+__global__ void __launch_bounds__(m3lb::kBlock) k_energy(m3lb::Dom d, m3lb::FastDiv div_nx,
+                                                         m3lb::FastDiv div_ny, const R* u,
+                                                         size_t comp, int zfirst, int z0, int z1,
+                                                         double* out) {
+  const unsigned N = unsigned(d.nx) * unsigned(d.ny) * unsigned(z1 - z0);
+  const R *ux = u, *uy = u + comp, *uz = u + 2 * comp;
+  double acc[3] = {0, 0, 0};
+  for (unsigned i = blockIdx.x * unsigned(m3lb::kBlock) + threadIdx.x; i < N;
+       i += gridDim.x * unsigned(m3lb::kBlock)) {
+    const unsigned row = m3lb::fd_div(div_nx, i), zz = m3lb::fd_div(div_ny, row);
+    const int x = int(i - row * unsigned(d.nx)), y = int(row - zz * unsigned(d.ny)), z = z0 + int(zz);
+    auto plane = [&](int zp) {
+      if (zfirst != kWholeBox) return zp - zfirst;
+      return (zp < 0 ? zp + d.nz : (zp >= d.nz ? zp - d.nz : zp)) + d.hz;
+    };
+    auto id = [&](int xx, int yy, int zp) {
+      xx = xx < 0 ? xx + d.nx : (xx >= d.nx ? xx - d.nx : xx);
+      yy = yy < 0 ? yy + d.ny : (yy >= d.ny ? yy - d.ny : yy);
+      return (plane(zp) * d.sy + (yy + d.hy)) * d.sx + xx + d.hx;
     };
     const int n = id(x, y, z);
     const double a = ux[n], b = uy[n], c = uz[n];
-    if (!isfinite(a) || !isfinite(b) || !isfinite(c)) { ok = false; continue; }
+    if (!isfinite(a) || !isfinite(b) || !isfinite(c)) { acc[2] += 1.0; continue; }
     acc[0] += 0.5 * (a * a + b * b + c * c);
-    const double wz = 0.5 * (uy[id(x + 1, y, z)] - uy[id(x - 1, y, z)]) -
-                      0.5 * (ux[id(x, y + 1, z)] - ux[id(x, y - 1, z)]);
+    const double wz = 0.5 * (double(uy[id(x + 1, y, z)]) - double(uy[id(x - 1, y, z)])) -
+                      0.5 * (double(ux[id(x, y + 1, z)]) - double(ux[id(x, y - 1, z)]));
     double wx = 0, wy = 0;
     if (d.nz > 1) {
-      wx = 0.5 * (uz[id(x, y + 1, z)] - uz[id(x, y - 1, z)]) -
-           0.5 * (uy[id(x, y, z + 1)] - uy[id(x, y, z - 1)]);
-      wy = 0.5 * (ux[id(x, y, z + 1)] - ux[id(x, y, z - 1)]) -
-           0.5 * (uz[id(x + 1, y, z)] - uz[id(x - 1, y, z)]);
+      wx = 0.5 * (double(uz[id(x, y + 1, z)]) - double(uz[id(x, y - 1, z)])) -
+           0.5 * (double(uy[id(x, y, z + 1)]) - double(uy[id(x, y, z - 1)]));
+      wy = 0.5 * (double(ux[id(x, y, z + 1)]) - double(ux[id(x, y, z - 1)])) -
+           0.5 * (double(uz[id(x + 1, y, z)]) - double(uz[id(x - 1, y, z)]));
     }
     acc[1] += 0.5 * (wx * wx + wy * wy + wz * wz);
   }
-  if (!ok) *finite = 0;
-  m3lb::block_sum<2>(acc, out);
+  m3lb::block_sum<3>(acc, out);
 }
 
 // Plain in-place stream, one float4 per thread: the best a memory-bound
@@ -1343,42 +1352,63 @@ extern "C" int m3lb_stream_probe(uint64_t bytes, int32_t nontemporal, int32_t re
 extern "C" int m3lb_energy_enstrophy(m3lb_solver* s, double* energy, double* enstrophy,
                                      int32_t* finite) {
   if (!s || !energy || !enstrophy) return fail(M3LB_EINVAL, "null argument");
-  const size_t np = size_t(s->d.np);
-  double* buf = nullptr;
-  int* fl = nullptr;
-  HIP_OK(hipMalloc(&buf, 3 * np * sizeof(double)));
-  HIP_OK(hipMalloc(&fl, sizeof(int)));
-  const int one = 1;
-  HIP_OK(hipMemcpyAsync(fl, &one, sizeof(int), hipMemcpyHostToDevice, s->stream));
+  // The velocities go through a scratch of at most kKeptWork bytes: the whole
+  // box, or slabs of planes with the planes beside them (the wrap included).
+  const m3lb::Dom& d = s->d;
+  const size_t rb = size_t(s->ks->real_bytes), plane = size_t(d.sx) * size_t(d.sy);
+  const size_t room = kKeptWork / (3 * plane * rb);
+  const bool whole = size_t(d.sz) <= room || d.nz < 4;
+  const int slab = whole ? d.nz : int(std::max<size_t>(3, room)) - 2;
+  const int slabs = (d.nz + slab - 1) / slab;
+  const size_t comp = plane * size_t(whole ? d.sz : slab + 2);
+  int rc = ensure_work(s, 3 * comp * rb);
+  const int64_t nodes = int64_t(d.nx) * d.ny * std::min(slab, d.nz);
+  // the partials of all slabs fit a staging slot
+  const unsigned cap = std::max(1u, std::min(4096u, 131072u / unsigned(slabs)));
+  const unsigned grid = std::max(1u, std::min(cap, m3lb::blocks_for(nodes)));
+  if (!rc) rc = ensure_partials(s, size_t(grid) * size_t(slabs) * 3);
+  if (rc) return rc;
   m3lb::ReadArgs a = read_args(s);
-  a.out2[0] = nullptr;
-  for (int k = 0; k < 3; ++k) a.out2[1 + k] = buf + k * np;
-  s->ks->macro(a, s->stream);
-  const long long N = (long long)s->d.nx * s->d.ny * s->d.nz;
-  const unsigned grid = std::max(1u, std::min(4096u, unsigned((N + m3lb::kBlock - 1) / m3lb::kBlock)));
-  int rc = ensure_partials(s, size_t(grid) * 2);
-  if (!rc) {
-    k_energy<<<grid, m3lb::kBlock, 0, s->stream>>>(s->d, buf, buf + np, buf + 2 * np, s->partial_d, fl);
+  char* buf = static_cast<char*>(s->work_d);
+  // velocities of interior planes [za, zb) to plane `at` of the scratch
+  auto velocities = [&](int za, int zb, int at) {
+    if (zb <= za) return;
+    a.n0 = whole ? 0 : int((za + d.hz) * int64_t(plane));
+    a.n1 = whole ? d.np : int((zb + d.hz) * int64_t(plane));
+    a.out2[0] = nullptr;
+    for (int k = 0; k < 3; ++k) a.out2[1 + k] = buf + (size_t(k) * comp + size_t(at) * plane) * rb;
+    s->ks->macro(a, s->stream);
+  };
+  const m3lb::FastDiv dx = m3lb::make_fastdiv(uint32_t(d.nx)), dy = m3lb::make_fastdiv(uint32_t(d.ny));
+  for (int k = 0; k < slabs && !rc; ++k) {
+    const int z0 = k * slab, z1 = std::min(d.nz, z0 + slab);
+    if (whole) {
+      velocities(0, d.nz, 0);
+    } else {
+      if (z0 == 0) velocities(d.nz - 1, d.nz, 0);
+      velocities(std::max(0, z0 - 1), std::min(d.nz, z1 + 1), z0 == 0 ? 1 : 0);
+      if (z1 == d.nz) velocities(0, 1, z1 - z0 + 1);
+    }
+    double* out = s->partial_d + size_t(k) * grid * 3;
+    const int zfirst = whole ? kWholeBox : z0 - 1;
+    if (rb == 8)
+      k_energy<double><<<grid, m3lb::kBlock, 0, s->stream>>>(
+          d, dx, dy, reinterpret_cast<const double*>(buf), comp, zfirst, z0, z1, out);
+    else
+      k_energy<float><<<grid, m3lb::kBlock, 0, s->stream>>>(
+          d, dx, dy, reinterpret_cast<const float*>(buf), comp, zfirst, z0, z1, out);
     rc = launch_ok();
   }
-  std::vector<double> h(size_t(grid) * 2);
-  int okv = 1;
-  if (!rc) {
-    if (hipMemcpyAsync(h.data(), s->partial_d, h.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-        hipMemcpyAsync(&okv, fl, sizeof(int), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-      rc = fail(M3LB_EDEVICE, "energy download failed");
-  }
-  hipError_t e = hipStreamSynchronize(s->stream);
-  hipFree(buf);
-  hipFree(fl);
+  double sums[3] = {0, 0, 0};
+  if (!rc)
+    rc = m3lb::read_column_sums(s->partial_d, grid * unsigned(slabs), 3, s->device, s->stream, sums);
+  const int sync_rc = stream_sync(s);  // reports a failed two-step pass
+  drop_work(s);
   if (rc) return rc;
-  if (e != hipSuccess) return fail(M3LB_EDEVICE, hipGetErrorString(e));
-  SYNC_OK(s);  // reports a failed two-step pass
-  double E = 0, W = 0;
-  for (unsigned b = 0; b < grid; ++b) { E += h[2 * b]; W += h[2 * b + 1]; }
-  *energy = E;
-  *enstrophy = W;
-  if (finite) *finite = okv;
+  if (sync_rc) return sync_rc;
+  *energy = sums[0];
+  *enstrophy = sums[1];
+  if (finite) *finite = sums[2] == 0.0 ? 1 : 0;
   return M3LB_OK;
 }
 
@@ -1386,20 +1416,8 @@ extern "C" {
 
 static int read_pops(m3lb_solver* s, double* out, bool logical) {
   if (!s || !out) return fail(M3LB_EINVAL, "null argument");
-  const size_t n = size_t(s->d.np) * size_t(s->Q);
-  double* buf = nullptr;
-  HIP_OK(hipMalloc(&buf, n * sizeof(double)));
-  m3lb::ReadArgs a = read_args(s);
-  a.out = buf;
-  if (logical) s->ks->gather(a, s->stream);
-  else s->ks->storage(a, s->stream);
-  int rc = launch_ok();
-  if (!rc && hipMemcpyAsync(out, buf, n * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-    rc = fail(M3LB_EDEVICE, "population download failed");
-  hipError_t e = hipStreamSynchronize(s->stream);
-  hipFree(buf);
+  const int rc = m3lb::read_populations(s->ks, read_args(s), s->Q, logical, s->device, s->stream, out);
   if (rc) return rc;
-  if (e != hipSuccess) return fail(M3LB_EDEVICE, hipGetErrorString(e));
   SYNC_OK(s);  // reports a failed two-step pass
   return M3LB_OK;
 }
