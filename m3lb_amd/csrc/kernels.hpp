@@ -508,8 +508,8 @@ __global__ void __launch_bounds__(kBlock) k_step_batched(BatchArgs a) {
 // padded box in ascending node order and writes population i of node n into
 // the slot load() reads, with neighbours clamped at non-periodic faces; where
 // clamping makes two nodes write one slot the later (higher-indexed) one is
-// what remains.  Here every slot is visited once and takes the value of its
-// highest-indexed writer, which is that same result with no write conflict.
+// what remains.  Here only a slot's highest-indexed writer writes it, which is
+// that same result with no write conflict.
 // ---------------------------------------------------------------------------
 enum SeedMode { kSeedUniform = 0, kSeedField = 1, kSeedArray = 2, kSeedTaylorGreen = 3 };
 
@@ -592,62 +592,45 @@ __device__ __forceinline__ void seed_value_of(const SeedArgs& a, int n, typename
   }
 }
 
+// One thread per padded node: its Q values are formed once (the analytic
+// fields cost FP64 sines and cosines, so evaluating a node again for each of
+// its 13 neighbours' slots made the kernel 14 times the work: 512^3 FP32
+// Taylor-Green 34 ms, now 5.5) and written into the slots load() reads, each by its
+// highest-indexed writer only.
 template <class K>
 __global__ void __launch_bounds__(kBlock) k_seed(SeedArgs a) {
   using R = typename K::R;
   using T = typename K::T;
   using C = typename K::C;
   constexpr int Q = K::Q;
-  const int m = blockIdx.x * kBlock + threadIdx.x;
+  const int n = blockIdx.x * kBlock + threadIdx.x;
   const Dom& d = a.d;
-  if (m >= d.np) return;
-  const int mx = m % d.sx, my = (m / d.sx) % d.sy, mz = m / (d.sx * d.sy);
+  if (n >= d.np) return;
+  const int x = n % d.sx, y = (n / d.sx) % d.sy, z = n / (d.sx * d.sy);
   T* A = static_cast<T*>(a.f);
-  R own[Q];
-  if (a.mode != kSeedArray) seed_value_of<K>(a, m, own);
-  sfor<Q>([&](auto Qs) {
-    constexpr int q = Qs;
-    // direction i written into slot q, and the displacement e with
-    // nbr(writer, e) == m for remote slots (EsotericPull.hpp:104-111)
-    int i = q, ex = 0, ey = 0, ez = 0;
-    bool remote = false;
-    if constexpr (q != 0) {
-      if (a.parity == 0) {
-        if constexpr ((q & 1) == 0) {
-          remote = true;
-          ex = Lat<Q>::cx[q - 1]; ey = Lat<Q>::cy[q - 1]; ez = Lat<Q>::cz[q - 1];
-        }
-      } else {
-        if constexpr ((q & 1) == 0) {
-          i = q - 1;
-        } else {
-          i = q + 1;
-          remote = true;
-          ex = Lat<Q>::cx[q]; ey = Lat<Q>::cy[q]; ez = Lat<Q>::cz[q];
-        }
-      }
-    }
-    int w = m;
-    if (remote) {
-      const int wx = writer_axis(mx, ex, d.nx, d.sx, d.px);
-      const int wy = writer_axis(my, ey, d.ny, d.sy, d.py);
-      const int wz = writer_axis(mz, ez, d.nz, d.sz, d.pz);
-      w = (wx < 0 || wy < 0 || wz < 0) ? -1 : (wz * d.sy + wy) * d.sx + wx;
-    }
-    if (w < 0) return;  // no node writes this slot: it keeps its value
-    R val;
-    if (a.mode == kSeedArray) {
-      val = static_cast<const R*>(a.arr)[uint64_t(w) * Q + i];
-    } else if (w == m) {
-      val = R(0);
-      sfor<Q>([&](auto J) { if (int(J) == i) val = own[int(J)]; });
-    } else {
-      R other[Q];
-      seed_value_of<K>(a, w, other);
-      val = R(0);
-      sfor<Q>([&](auto J) { if (int(J) == i) val = other[int(J)]; });
-    }
-    A[uint64_t(q) * a.stride + unsigned(m)] = C::enc(val, a.scale[q]);
+  R v[Q];
+  if (a.mode == kSeedArray)
+    sfor<Q>([&](auto I) { v[int(I)] = static_cast<const R*>(a.arr)[uint64_t(n) * Q + int(I)]; });
+  else
+    seed_value_of<K>(a, n, v);
+  A[unsigned(n)] = C::enc(v[0], a.scale[0]);
+  // only nodes at the last layers of an axis without wrap share a slot
+  const bool edge = (!d.px && (x < 2 || x > d.sx - 3)) || (!d.py && (y < 2 || y > d.sy - 3)) ||
+                    (!d.pz && (z < 2 || z > d.sz - 3));
+  sfor<(Q - 1) / 2>([&](auto Pr) {
+    constexpr int i = 2 * Pr + 1;  // i: the node's own slot; i + 1: its neighbour's
+    constexpr int ex = Lat<Q>::cx[i], ey = Lat<Q>::cy[i], ez = Lat<Q>::cz[i];
+    const int own = a.parity == 0 ? i : i + 1, nbr = a.parity == 0 ? i + 1 : i;
+    A[uint64_t(own) * a.stride + unsigned(n)] = C::enc(v[i], a.scale[own]);
+    const int mx = shift_axis(x + ex, d.hx, d.nx, d.sx, d.px);
+    const int my = shift_axis(y + ey, d.hy, d.ny, d.sy, d.py);
+    const int mz = shift_axis(z + ez, d.hz, d.nz, d.sz, d.pz);
+    if (edge && (writer_axis(mx, ex, d.nx, d.sx, d.px) != x ||
+                 writer_axis(my, ey, d.ny, d.sy, d.py) != y ||
+                 writer_axis(mz, ez, d.nz, d.sz, d.pz) != z))
+      return;
+    A[uint64_t(nbr) * a.stride + unsigned((mz * d.sy + my) * d.sx + mx)] =
+        C::enc(v[i + 1], a.scale[nbr]);
   });
 }
 
