@@ -953,8 +953,10 @@ __device__ __forceinline__ void bc_partition(const typename K::R* f, const int n
   sfor<K::Q>([&](auto I) {
     constexpr int i = I;
     const int cn = cvel<K::Q>(i, 0) * nrm[0] + cvel<K::Q>(i, 1) * nrm[1] + cvel<K::Q>(i, 2) * nrm[2];
-    if (cn > 0) out += f[i];
-    else if (cn == 0) tang += f[i];
+    // two selects: as a branch the compiler picks the sum to add to by its
+    // address, which puts both into scratch memory, one round trip a direction
+    out = cn > 0 ? out + f[i] : out;
+    tang = cn == 0 ? tang + f[i] : tang;
   });
 }
 template <class K>

@@ -44,10 +44,12 @@ struct KernelSet {
 };
 
 // Regions of the plane kernel (PlaneArgs) and what moves in the box.
-enum PlaneRegion { kPlaneSquare = 0, kPlaneWide = 1 };
+enum PlaneRegion { kPlaneSquare = 0, kPlaneWide = 1, kPlaneSmall = 2 };
 enum PlaneNodes { kPlaneFluid = 0, kPlaneGeom = 1, kPlaneWalls = 2 };
 using PlaneSquare = PlaneShape<32, 32, 1024>;
 using PlaneWide = PlaneShape<64, 32, 512>;
+using PlaneSmall = PlaneShape<24, 24, 576>;
+using PlaneWalled = PlaneShape<32, 28, 896, true>;
 
 inline unsigned blocks_for(long long n) { return unsigned((n + kBlock - 1) / kBlock); }
 
@@ -164,9 +166,12 @@ struct Launch {
   static void plane(const PlaneArgs& a, int shape, int nodes, hipStream_t s) {
     if constexpr (kPlane) {
       if (nodes == kPlaneWalls) {
-        if constexpr (K::OP != M3LB_OP_NULL)
-          k_plane<K, PlaneSquare, true, true>
-              <<<unsigned(a.ntx) * unsigned(a.nty), PlaneSquare::NT, 0, s>>>(a);
+        if constexpr (K::OP != M3LB_OP_NULL) {
+          k_plane<K, PlaneWalled, true, true>
+              <<<unsigned(a.ntx) * unsigned(a.nty), PlaneWalled::NT, 0, s>>>(a);
+        }
+      } else if (shape == kPlaneSmall) {
+        plane_s<PlaneSmall>(a, nodes, s);
       } else if (shape == kPlaneSquare) {
         plane_s<PlaneSquare>(a, nodes, s);
       } else {

@@ -33,15 +33,17 @@ struct PlaneArgs {
   StepArgs a;
   void* out;      // the other population array
   int ntx, nty;   // blocks along x and y
+  int core_x, more_x, core_y, more_y;  // sx / ntx, sx % ntx, sy / nty, sy % nty
   int steps;      // T, even
   int margin;     // H: T, with walls T + 2
   WallArgs w;     // WALLS only
 };
 
-// RX x RY nodes per region, NT threads.
-template <int RX_, int RY_, int NT_>
+// RX x RY nodes per region; NF threads take the fluid cells and, with walls, two
+// more waves the straight wall cells and the corners.
+template <int RX_, int RY_, int NF_, bool WAVES_ = false>
 struct PlaneShape {
-  static constexpr int RX = RX_, RY = RY_, NT = NT_;
+  static constexpr int RX = RX_, RY = RY_, NF = NF_, NW = WAVES_ ? 128 : 0, NT = NF + NW;
 };
 
 // What a block keeps of its wall cells, so that a step reads no tables: the
@@ -49,12 +51,14 @@ struct PlaneShape {
 // for corners this step's extrapolated density and the gradient sums
 // (d_x u, d_y v, d_x v + d_y u) of the finite-difference stress.  list: the
 // wall cells, straight ones from the front, corners from the back.  A step's
-// wall code is a long chain that one wave runs for a whole list (a wall along
-// y has one cell in each row: updated with the rows, every wave would run it
-// for one or two lanes), the first wave for the straight cells and the last one
-// for the corners, beside the fluid cells.  Cavity 129^2 FP64: 9.3 us per step
-// with the rows, 5.8 with the list (18.4 one launch at a time); 0.9 of it are the
-// fluid cells, 1.4 the straight ones, 2.3 the corners and their densities.
+// wall code is a long chain, bound by the rate at which one wave issues it (800
+// instructions for a straight cell): one wave runs it for all straight cells of
+// the region and another one for the corners, beside the waves of the fluid
+// cells.  Cavity 129^2 FP64 CM, us per step: 18.4 one launch at a time; 9.3 with
+// the wall cells updated with the rows (every wave then runs the chain for one
+// or two lanes); 5.8 with waves that take fluid cells as well; 4.0 with waves of
+// their own and the closure sums out of scratch memory; 3.7 with the corners'
+// densities beside the other cells' work.
 template <class R, int N, bool WALLS>
 struct PlaneWalls {
   R u[3][N];
@@ -137,8 +141,9 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
   using T = typename K::T;
   using C = typename K::C;
   constexpr int Q = K::Q, RX = S::RX, RY = S::RY, NP = RX * RY;
-  constexpr int kPerThread = (NP + S::NT - 1) / S::NT;
-  static_assert(NP % S::NT == 0 && (RX & (RX - 1)) == 0, "whole rounds of threads");
+  constexpr int kPerThread = NP / S::NF;
+  static_assert(NP % S::NF == 0 && S::NF % 64 == 0, "whole rounds of threads and waves");
+  static_assert(!WALLS || S::NW == 128, "walls have two waves of their own");
   __shared__ T s[Q * NP];
   __shared__ PlaneWalls<R, NP, WALLS> pw;
   const StepArgs& a = pa.a;
@@ -146,8 +151,9 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
   const int H = pa.margin;
   const unsigned tile = tile_of(blockIdx.x, gridDim.x, a.remap);
   const int ity = int(tile / unsigned(pa.ntx)), itx = int(tile - unsigned(ity) * unsigned(pa.ntx));
-  const int X0 = int(int64_t(itx) * d.sx / pa.ntx), X1 = int(int64_t(itx + 1) * d.sx / pa.ntx);
-  const int Y0 = int(int64_t(ity) * d.sy / pa.nty), Y1 = int(int64_t(ity + 1) * d.sy / pa.nty);
+  // cores of core_x or core_x + 1 nodes, the first more_x of them the larger
+  const int X0 = itx * pa.core_x + min(itx, pa.more_x), X1 = X0 + pa.core_x + (itx < pa.more_x);
+  const int Y0 = ity * pa.core_y + min(ity, pa.more_y), Y1 = Y0 + pa.core_y + (ity < pa.more_y);
   const Params<R> p = params_of<K>(a);
   const T* A = static_cast<const T*>(a.f);
   T* B = static_cast<T*>(pa.out);
@@ -195,10 +201,11 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
   };
 
   // ---- step 0: source array to LDS ----
+  const bool fluid_wave = S::NW == 0 || int(threadIdx.x) < S::NF;
   uint32_t moves = 0;  // bit j: this thread's j-th cell is fluid
 #pragma unroll 1
-  for (int j = 0; j < kPerThread; ++j) {
-    const int c = int(threadIdx.x) + j * S::NT;
+  for (int j = 0; fluid_wave && j < kPerThread; ++j) {
+    const int c = int(threadIdx.x) + j * S::NF;
     int X, Y;
     if (!within(c, H - 1) || !cell_xy(c, X, Y)) continue;
     const int n = Y * d.sx + X, x = X - d.hx, y = Y - d.hy;
@@ -268,6 +275,7 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
   }
   __syncthreads();
   int nstraight = 0, ncorner = 0;
+  const int wall_lane = int(threadIdx.x) - S::NF;  // negative in the fluid waves
   if constexpr (WALLS) {
     nstraight = pw.straight;
     ncorner = pw.corners;
@@ -277,14 +285,12 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
   // outgrows the instruction cache).  Opposite directions share their scale.
   auto wall_cells = [&](int t, int k) {
     if constexpr (WALLS) {
+      if (fluid_wave) return;
       const int pp = t & 1;
+      const bool corner = wall_lane >= 64;
 #pragma unroll 1
-      for (int w = int(threadIdx.x); w < NP; w += S::NT) {
-        // straight cells from the first thread on, corners from the last one
-        const int v = NP - 1 - w;
-        if (w >= nstraight && v >= ncorner) continue;
-        const bool corner = v < ncorner;
-        const int c = pw.list[w];
+      for (int w = wall_lane & 63; w < (corner ? ncorner : nstraight); w += 64) {
+        const int c = pw.list[corner ? NP - 1 - w : w];
         if (!within(c, k)) continue;
         R f[Q];
         int X, Y;
@@ -320,45 +326,70 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
     }
   };
 
-  // corners first: their stencils read slots that other nodes update
+  // corners first: their stencils read slots that other nodes update.  Two
+  // lanes take the two closure densities of a corner's stencil.  Up to 32
+  // corners are read before the barrier and worked on after it, beside the
+  // straight and the fluid cells.
   auto corners = [&](int t, int k) {
     if constexpr (WALLS) {
       if (ncorner == 0) return;
       const int pp = t & 1;
-#pragma unroll 1
-      for (int v = S::NT - 1 - int(threadIdx.x); v < ncorner; v += S::NT) {
-        const int c = pw.list[NP - 1 - v];
-        const uint32_t info = pw.info[c];
-        if (!within(c, k)) continue;
-        const R rho = corner_rho(info, [&](int steps, int ax) -> R {
-          int cm = c + steps * (ax == 0 ? 1 : RX);
-          // beyond the region: a corner that no core node sees in T steps
-          if (cm < RX + 1 || cm >= NP - RX - 1) cm = c;
-          R g[Q];
-          g[0] = C::dec(s[cm], a.inv_scale[0]);
-          sfor<(Q - 1) / 2>([&](auto Pr) {
-            constexpr int i = 2 * Pr + 1;
-            g[i] = C::dec(s[(i + pp) * NP + cm], a.inv_scale[i]);
-            g[i + 1] = C::dec(s[(i + 1 - pp) * NP + cm + cvel<Q>(i, 1) * RX + cvel<Q>(i, 0)],
-                              a.inv_scale[i]);
-          });
-          const R u[3] = {pw.u[0][cm], pw.u[1][cm], pw.u[2][cm]};
-          return density_of(g, int(pw.info[cm] & 15u), u);
+      R g[Q];
+      int c = 0, cm = 0, e = 0;
+      auto read = [&](int v) {  // every lane of the wave stays for the exchange below
+        c = pw.list[NP - 1 - (v < ncorner ? v : 0)];
+        e = int(pw.info[c] >> 4 & 15u);
+        const int reach = ((e & 1) ? 1 : -1) * (1 + (wall_lane & 1));
+        cm = c + (e == 0 ? 0 : reach * ((e - 1) >> 1 == 0 ? 1 : RX));
+        // beyond the region: a corner that no core node sees in T steps
+        if (cm < RX + 1 || cm >= NP - RX - 1) cm = c;
+        g[0] = C::dec(s[cm], a.inv_scale[0]);
+        sfor<(Q - 1) / 2>([&](auto Pr) {
+          constexpr int i = 2 * Pr + 1;
+          g[i] = C::dec(s[(i + pp) * NP + cm], a.inv_scale[i]);
+          g[i + 1] = C::dec(s[(i + 1 - pp) * NP + cm + cvel<Q>(i, 1) * RX + cvel<Q>(i, 0)],
+                            a.inv_scale[i]);
         });
-        pw.rho[c] = rho;
-        if (t == pa.steps - 1) {
-          int X, Y;
-          (void)cell_xy(c, X, Y);
-          static_cast<R*>(pa.w.bc_rho)[Y * d.sx + X] = rho;
+      };
+      auto finish = [&](int v) {
+        const R u[3] = {pw.u[0][cm], pw.u[1][cm], pw.u[2][cm]};
+        const R r1 = density_of(g, int(pw.info[cm] & 15u), u);
+        const R r2 = __shfl_xor(r1, 1);
+        if (!(wall_lane & 1) && v < ncorner && within(c, k)) {
+          const R rho = e != 0 ? R(2) * r1 - r2 : R(1);
+          pw.rho[c] = rho;
+          if (t == pa.steps - 1) {
+            int X, Y;
+            (void)cell_xy(c, X, Y);
+            static_cast<R*>(pa.w.bc_rho)[Y * d.sx + X] = rho;
+          }
+        }
+      };
+      const bool mine = wall_lane >= 64;
+      const int v = (wall_lane & 63) >> 1;
+      if (mine) {
+        read(v);
+        if (ncorner > 32) {
+          finish(v);
+#pragma unroll 1
+          for (int v0 = 32; v0 < ncorner; v0 += 32) {
+            read(v0 + v);
+            finish(v0 + v);
+          }
         }
       }
       __syncthreads();
+      if (mine && ncorner <= 32) {
+        finish(v);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read by this wave's lanes
+        __builtin_amdgcn_wave_barrier();
+      }
     }
   };
   auto fluid_cells = [&](auto PP, int k) {
 #pragma unroll 1
     for (int j = 0; j < kPerThread; ++j) {
-      const int c = int(threadIdx.x) + j * S::NT;
+      const int c = int(threadIdx.x) + j * S::NF;
       if (!(moves >> j & 1u) || !within(c, k)) continue;
       R f[Q];
       lds_load<K, int(PP)>(s, NP, c, RX, a.inv_scale, f);
@@ -398,8 +429,8 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
                             offsets(d, X - d.hx, Y - d.hy, 0), a.scale, f);
   };
 #pragma unroll 1
-  for (int j = 0; j < kPerThread; ++j) {
-    const int c = int(threadIdx.x) + j * S::NT;
+  for (int j = 0; fluid_wave && j < kPerThread; ++j) {
+    const int c = int(threadIdx.x) + j * S::NF;
     if (!within(c, 0)) continue;
     if (moves >> j & 1u) {
       R f[Q];

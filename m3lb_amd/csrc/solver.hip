@@ -836,15 +836,33 @@ struct PlanePlan {
   int shape = 0, nodes = 0;
 };
 
-// Region and steps per launch.  A plane that 32 x 32 regions cover in one
-// round of blocks at 8 steps is bound by launches and by the latency of a
-// step: 8 steps per launch (D2Q9 128^2: FP32 1.28 us per step against 1.5 at
-// 6, 1.8 at 4 and 2.75 one launch per step; FP64 1.40 against 3.0).  Larger
-// ones are bound by traffic and by the work on margins: 4-byte and 2-byte
-// populations take 64 x 32 regions and 6 steps (1024^2 FP32 7.9 us per step,
-// 8.0 at 4 steps, 9.3 with 32 x 32 regions, 11.1 one launch per step; 4096^2
-// 93, 96, 125 and 189), 8-byte ones 32 x 32 and 4 (1024^2 12.0 us, 12.2 at 6,
-// 13.5 with 64 x 32 regions, 23.6 one launch per step; 4096^2 169 and 426).
+int plane_margin(int steps, int nodes) { return steps + (nodes == m3lb::kPlaneWalls ? 2 : 0); }
+struct PlaneRegionSize {
+  int x, y;
+};
+PlaneRegionSize region_size(int shape, int nodes) {
+  using namespace m3lb;
+  if (nodes == kPlaneWalls) return {PlaneWalled::RX, PlaneWalled::RY};
+  if (shape == kPlaneSmall) return {PlaneSmall::RX, PlaneSmall::RY};
+  if (shape == kPlaneWide) return {PlaneWide::RX, PlaneWide::RY};
+  return {PlaneSquare::RX, PlaneSquare::RY};
+}
+
+// Region and steps per launch.  While the blocks of a region fit the chip in
+// one round, a launch lasts as long as one block: the most steps that still
+// fit, in the smallest region (fewer nodes of margin per wave).  us per step,
+// FP64 BGK / FP32 CM:
+//   128^2  24 x 24 regions, 8 steps 1.17 / 1.05; 32 x 32, 8 1.34 / 1.21
+//   192^2  24 x 24, 6 1.42 / 1.24;  32 x 32, 8 1.50 / 1.32
+//   256^2  32 x 32, 8 1.67 / 1.41;  6 steps 1.80 / 1.56
+//   320^2  32 x 32, 6 1.95 / 1.63;  8 steps (two rounds) 2.76 / 2.16
+//   384^2  32 x 32, 4 2.41 / 2.09;  6 steps 2.98 / 2.47, 8 3.67 / 2.95
+// with walls (cavity FP64 CM): 129^2 8 steps 3.7, 6 3.8, 4 4.5; 257^2 4.7, 5.6, 7.8.
+// Larger planes are bound by traffic and by the work on margins: 4-byte and
+// 2-byte populations take 64 x 32 regions and 6 steps (1024^2 FP32 7.9 us per
+// step, 8.0 at 4 steps, 9.3 with 32 x 32 regions, 11.1 one launch per step;
+// 4096^2 93, 96, 125 and 189), 8-byte ones 32 x 32 and 4 (1024^2 12.0 us, 12.2
+// at 6, 13.5 with 64 x 32 regions, 23.6 one launch per step; 4096^2 169 and 426).
 PlanePlan plane_plan(const m3lb_solver* s) {
   PlanePlan p;
   const Boundaries& b = s->b;
@@ -855,12 +873,20 @@ PlanePlan plane_plan(const m3lb_solver* s) {
   if (!(d.px || d.hx) || !(d.py || d.hy)) return p;
   p.nodes = b.nwall ? m3lb::kPlaneWalls
                     : (s->geometry || d.hx || d.hy ? m3lb::kPlaneGeom : m3lb::kPlaneFluid);
-  const int core8 = m3lb::PlaneSquare::RX - 2 * (b.nwall ? 10 : 8);
-  const int64_t blocks8 = int64_t((d.sx + core8 - 1) / core8) * ((d.sy + core8 - 1) / core8);
+  const int steps_shapes[5][2] = {{8, m3lb::kPlaneSmall},  {6, m3lb::kPlaneSmall},
+                                  {8, m3lb::kPlaneSquare}, {6, m3lb::kPlaneSquare},
+                                  {4, m3lb::kPlaneSquare}};
+  for (const auto& c : steps_shapes) {
+    if (b.nwall && c[1] == m3lb::kPlaneSmall) continue;
+    const PlaneRegionSize r = region_size(c[1], p.nodes);
+    const int h = plane_margin(c[0], p.nodes), cx = r.x - 2 * h, cy = r.y - 2 * h;
+    if (int64_t((d.sx + cx - 1) / cx) * ((d.sy + cy - 1) / cy) > s->cus) continue;
+    p.steps = c[0];
+    p.shape = c[1];
+    return p;
+  }
   p.shape = m3lb::kPlaneSquare;
-  if (blocks8 <= (b.nwall ? 1 : 2) * int64_t(s->cus)) {
-    p.steps = 8;
-  } else if (b.nwall || s->ks->elem_bytes == 8) {
+  if (b.nwall || s->ks->elem_bytes == 8) {
     p.steps = 4;
   } else {
     p.shape = m3lb::kPlaneWide;
@@ -878,12 +904,15 @@ PlanePlan plane_plan(const m3lb_solver* s) {
 }
 
 // The second population array: allocated at the first pass, and given the
-// slots no moving node writes whenever those may have changed.  A failed
-// allocation leaves the box to one launch per step.
+// slots no moving node writes whenever those may have changed.  Where there is
+// no room for it the box is left to one launch per step.
 int ensure_alt(m3lb_solver* s, bool statics) {
   const size_t bytes = size_t(s->stride) * size_t(s->Q) * size_t(s->ks->elem_bytes);
   if (!s->f_alt) {
-    if (hipMalloc(&s->f_alt, bytes) != hipSuccess) {
+    // at most a quarter of what is free: other boxes keep room of their own
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || bytes > free_b / 4 ||
+        hipMalloc(&s->f_alt, bytes) != hipSuccess) {
       (void)hipGetLastError();
       s->f_alt = nullptr;
       s->alt_failed = true;
@@ -908,12 +937,15 @@ int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& 
   pa.w = wa;
   pa.out = s->f_alt;
   pa.steps = steps;
-  pa.margin = steps + (p.nodes == m3lb::kPlaneWalls ? 2 : 0);
-  const bool wide = p.shape == m3lb::kPlaneWide;
-  const int cx = (wide ? m3lb::PlaneWide::RX : m3lb::PlaneSquare::RX) - 2 * pa.margin;
-  const int cy = (wide ? m3lb::PlaneWide::RY : m3lb::PlaneSquare::RY) - 2 * pa.margin;
+  pa.margin = plane_margin(steps, p.nodes);
+  const PlaneRegionSize r = region_size(p.shape, p.nodes);
+  const int cx = r.x - 2 * pa.margin, cy = r.y - 2 * pa.margin;
   pa.ntx = (s->d.sx + cx - 1) / cx;
   pa.nty = (s->d.sy + cy - 1) / cy;
+  pa.core_x = s->d.sx / pa.ntx;
+  pa.more_x = s->d.sx % pa.ntx;
+  pa.core_y = s->d.sy / pa.nty;
+  pa.more_y = s->d.sy % pa.nty;
   s->ks->plane(pa, p.shape, p.nodes, s->stream);
   std::swap(s->f, s->f_alt);
   return launch_ok();

@@ -208,3 +208,37 @@ def test_plane_wall_variants(variant):
                 s.set_wall_velocity_field_scale(1.3)
         s.initialize_field(*noise(cfg))
     images(cfg, setup, passes=variant != "outlet")
+
+
+@pytest.mark.parametrize("n,walls", [(128, False), (129, False), (192, False), (193, False),
+                                     (300, False), (385, False), (128, True), (129, True),
+                                     (192, True), (193, True), (257, True)])
+@pytest.mark.parametrize("dtype", [abi.F64, abi.F32])
+def test_plane_at_the_steps_of_the_rule(n, walls, dtype):
+    """Both sides of the sizes where the region or the steps per launch change."""
+    shape = (n, n - 1, 1)
+    cfg = abi.make_config(abi.D2Q9, abi.OP_CM, abi.SHIFTED, dtype, (n, n, 1) if walls else shape,
+                          periodic=(not walls, not walls, True), omega=1.6)
+
+    def setup(s):
+        if walls:
+            s.set_regularized_walls(*cases.cavity_walls(n, 0.05))
+        s.initialize_field(*noise(cfg))
+    images(cfg, setup, chunks=[1, 9, 22])
+
+
+def test_plane_many_corners():
+    """More corners per region than one wave takes at once."""
+    shape = (70, 36, 1)
+    nx, ny, _ = shape
+    cfg = abi.make_config(abi.D2Q9, abi.OP_CM, abi.SHIFTED, abi.F64, shape, periodic=(1, 0, 1),
+                          omega=1.2)
+    nrm = np.zeros((ny, nx), dtype=np.uint8)
+    nrm[0], nrm[-1] = cases.NRM_YM, cases.NRM_YP
+    nrm[4:-4:2, 3:-3:2] = cases.NRM_CORNER
+
+    def setup(s):
+        s.set_regularized_walls(nrm, np.zeros((ny, nx), dtype=np.uint16), np.zeros((1, 4)))
+        s.set_fd_corners(False)
+        s.initialize_field(*noise(cfg))
+    images(cfg, setup, chunks=[1, 9, 2])
