@@ -469,6 +469,37 @@ int rebuild_plan(m3lb_solver* s) {
     b.local = b.local && b.nrm[walls[w]] <= m3lb::kNrmCorner;
     for (int64_t r : reads[w]) b.local = b.local && r < 0;
   }
+  // A corner's density comes from two nodes along an axis, so a value travels
+  // two nodes further than one per step there.  The plane passes allow for that
+  // once: a value must not meet a second corner that takes it on in the same
+  // direction.  Corners of one direction lie at one coordinate along it, or
+  // further apart than a pass reaches.
+  constexpr int kReach = 32;
+  struct Ext {
+    int e, c[2];
+  };
+  std::vector<Ext> corners;
+  for (unsigned n : walls) {
+    if (!b.local || b.nrm[n] != m3lb::kNrmCorner || b.ext[n] == 0) continue;
+    int x, y, z;
+    coords(n, x, y, z);
+    const Ext q{int(b.ext[n]), {x, y}};
+    const int ax = (q.e - 1) >> 1;
+    b.local = ax < 2 && corners.size() < 256 &&
+              !((ax == 0 ? d.px : d.py) && (ax == 0 ? d.nx : d.ny) < 2 * kReach);
+    for (const Ext& o : corners) {
+      if (o.e != q.e || o.c[ax] == q.c[ax]) continue;
+      int far = 0;
+      for (int k = 0; k < 2; ++k) {
+        const int len = k == 0 ? d.nx : d.ny;
+        int dist = std::abs(o.c[k] - q.c[k]);
+        if (k == 0 ? d.px : d.py) dist = std::min(dist, len - dist);
+        far = std::max(far, dist);
+      }
+      b.local = b.local && far >= kReach;
+    }
+    corners.push_back(q);
+  }
   int rc = upload(b.wlist_d, wlist, s->stream);
   if (!rc) rc = upload(b.slist_d, spec, s->stream);
   if (!rc) rc = upload(b.snap_nodes_d, snap_nodes, s->stream);

@@ -227,18 +227,24 @@ def test_plane_at_the_steps_of_the_rule(n, walls, dtype):
     images(cfg, setup, chunks=[1, 9, 22])
 
 
-def test_plane_many_corners():
-    """More corners per region than one wave takes at once."""
+@pytest.mark.parametrize("chain", [False, True])
+def test_plane_many_corners(chain):
+    """More corners per region than one wave takes at once, and corners whose
+    stencils follow one another along an axis (one launch per step)."""
     shape = (70, 36, 1)
     nx, ny, _ = shape
     cfg = abi.make_config(abi.D2Q9, abi.OP_CM, abi.SHIFTED, abi.F64, shape, periodic=(1, 0, 1),
                           omega=1.2)
     nrm = np.zeros((ny, nx), dtype=np.uint8)
     nrm[0], nrm[-1] = cases.NRM_YM, cases.NRM_YP
-    nrm[4:-4:2, 3:-3:2] = cases.NRM_CORNER
+    if chain:
+        nrm[8, 20:30] = cases.NRM_YM
+        nrm[8, 20:30:3] = cases.NRM_CORNER
+    else:
+        nrm[4:-4:2, 3:-3:2] = cases.NRM_CORNER
 
     def setup(s):
         s.set_regularized_walls(nrm, np.zeros((ny, nx), dtype=np.uint16), np.zeros((1, 4)))
         s.set_fd_corners(False)
         s.initialize_field(*noise(cfg))
-    images(cfg, setup, chunks=[1, 9, 2])
+    images(cfg, setup, chunks=[1, 9, 2], passes=not chain)
