@@ -508,7 +508,7 @@ def main():
     # These counters see requests that the memory-side 256 MB cache serves as
     # well as those that reach HBM.
     traffic, traffic_src = None, None
-    tj = os.path.join(ROOT, "profiles", "k_pair_cm_f32_512cubed_traffic.json")
+    tj = os.path.join(ROOT, "profiles", "k_march_cm_f32_512cubed_traffic.json")
     build = solver.kernel_build_id()
     if args.size == 512 and args.dtype == "f32" and args.fusion != "off" and os.path.exists(tj):
         with open(tj) as fh:

@@ -317,7 +317,12 @@ int m3lb_set_tile_order(m3lb_solver* s, int32_t run);
 enum { M3LB_CACHE_AUTO = 0, M3LB_CACHE_STREAM = 1, M3LB_CACHE_PLAIN = 2 };
 int m3lb_set_cache_policy(m3lb_solver* s, int32_t policy);
 
-/* Two steps in one pass over the population array.  Step t+1 follows step t
+/* Two steps in one pass over the population array.  By default the steps of an
+ * FP32 or FP64 D3Q27 box beyond the last-level cache (CM, MRT, BGK with the
+ * product equilibrium; no per-node force) run through LDS into a
+ * second array of the same size (held from the first pass on, where a quarter of
+ * the free device memory has room for it); the values below tune the pass used
+ * where that one does not apply or any of them is set.  There step t+1 follows step t
  * a few z-planes behind inside one persistent launch, so that it reads step
  * t's output from the caches, and a short second launch finishes the rows
  * whose neighbours another stripe of the box updates: a pair of steps then
@@ -355,6 +360,9 @@ int m3lb_fused_passes(const m3lb_solver* s, uint64_t* passes);
  * and the next synchronising call reports M3LB_EDEVICE.  Never set outside
  * tests of that error path; off by default. */
 int m3lb_test_fail_fused_waits(m3lb_solver* s, int32_t on);
+/* Test hook: with on != 0 M3LB_FUSION_AUTO runs the passes through LDS on every
+ * box that their kernels take, whatever its size. */
+int m3lb_test_march_always(m3lb_solver* s, int32_t on);
 
 /* The block -> tile map the step kernel uses for `grid` blocks and a tile
  * order `run` (host-side copy of the device function): out[b] = tile of block

@@ -7,6 +7,7 @@
 #pragma once
 
 #include "kernels.hpp"
+#include "march.hpp"
 #include "pair.hpp"
 #include "plane.hpp"
 
@@ -41,6 +42,9 @@ struct KernelSet {
   // several steps of a plane box in one launch (plane.hpp); null where not
   // instantiated (D3Q27, per-node force)
   void (*plane)(const PlaneArgs&, int shape, int nodes, hipStream_t);
+  // two steps in one pass through LDS (march.hpp); null where not instantiated
+  // (D2Q9, 16-bit storage, per-node force, some operators)
+  void (*march)(const MarchArgs&, bool geom, hipStream_t);
 };
 
 // Regions of the plane kernel (PlaneArgs) and what moves in the box.
@@ -180,6 +184,20 @@ struct Launch {
       }
     }
   }
+  // BGK of second order and TRT compile to other fused multiply-adds in k_march
+  // than in k_step (results one rounding apart); they keep the pass of pair.hpp,
+  // whose bits are those of one launch per step.
+  static constexpr bool kMarch =
+      K::Q == 27 && !K::FIELD && !K::C::scaled &&
+      (K::OP == M3LB_OP_BGK_PRODUCT || K::OP == M3LB_OP_MRT || K::OP == M3LB_OP_CM);
+  static void march(const MarchArgs& a, bool geom, hipStream_t s) {
+    if constexpr (kMarch) {
+      const unsigned grid = unsigned(a.ntx) * unsigned(a.nty) * unsigned(a.nzc);
+      constexpr int nt = MarchShape<typename K::T>::NT;
+      if (geom) k_march<K, true><<<grid, nt, 0, s>>>(a);
+      else k_march<K, false><<<grid, nt, 0, s>>>(a);
+    }
+  }
   static void batched(const BatchArgs& a, unsigned grid, hipStream_t s) {
     if constexpr (kBatched) {
       if (a.run == kRunBlockRanges) {
@@ -199,7 +217,7 @@ struct Launch {
                                 kBatched ? batched : nullptr,
                                 kPair ? pair : nullptr,
                                 int(sizeof(typename K::T)), int(sizeof(typename K::R)),
-                                kPlane ? plane : nullptr};
+                                kPlane ? plane : nullptr, kMarch ? march : nullptr};
     return &t;
   }
 };

@@ -164,6 +164,7 @@ struct m3lb_solver {
   unsigned* pair_err_h = nullptr; // pinned: a failed wait in a pass, set by the tail launch
   uint64_t pair_passes = 0;       // pairs of steps run as one pass
   bool pair_fail_test = false;    // every wait of a pass gives up (failure-path test)
+  bool march_test = false;        // the march passes whatever the box (test)
 };
 
 namespace {
@@ -803,7 +804,8 @@ int pair_lag(const m3lb_solver* s) {
   return std::max(1, std::min(want, s->d.nz - 3));  // any lag in 1 .. nz-3 is exact
 }
 
-// The two-step pass applies when its kernels exist for this configuration,
+// The two-step pass in place (pair.hpp), where the one through LDS (march_plan
+// below) does not run.  It applies when its kernels exist for this configuration,
 // no boundary kernel has to run between the steps, the box has room for the
 // stripes and the lag, and (in AUTO) the populations exceed the last-level
 // cache, where the pass saves HBM traffic, in 4- or 8-byte storage.  Measured
@@ -982,6 +984,70 @@ int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& 
   return launch_ok();
 }
 
+// Two steps per pass through LDS (march.hpp).  The blocks along z are chosen for
+// the least rounds of blocks times planes of one (two planes and about half a
+// plane's time of start are extra).  It applies beyond the caches (within them a
+// step is bound by its arithmetic and loses to the margins: D3Q27 CM FP32 128^3
+// 28.1 GLUPS against 30.8) and where that schedule keeps the chip's cells filled:
+// 4-byte storage gains from 0.76 on (192^3 35.5 against 29.6 for the pass of
+// pair.hpp; 0.62, 160^3: 28.3 against 28.9), 8-byte from 0.55 (150x130x140 16.1
+// against 13.0).  It needs a second population array; where there is no room for
+// one, or the caller set the tuning values of pair.hpp, that pass runs.
+struct MarchPlan {
+  bool on = false;
+  int ntx = 0, nty = 0, nzc = 0;
+};
+MarchPlan march_plan(const m3lb_solver* s, const m3lb::StepArgs& a) {
+  MarchPlan p;
+  const m3lb::Dom& d = s->d;
+  if (!s->ks->march || s->fusion != M3LB_FUSION_AUTO || s->alt_failed) return p;
+  if (s->b.nwall || s->b.nspec || s->b.nsnap) return p;
+  if (!s->march_test &&
+      (a.cached || s->pair_stripes || s->pair_lag || s->pair_bpc || s->pair_group))
+    return p;
+  // an unwrapped axis without a halo (one node, not periodic) has no margin
+  if (!(d.px || d.hx) || !(d.py || d.hy) || !(d.pz || d.hz)) return p;
+  const bool wide = s->ks->elem_bytes == 8;
+  const int cx = wide ? m3lb::MarchShape<double>::W : m3lb::MarchShape<float>::W;
+  const int cy = wide ? m3lb::MarchShape<double>::CY : m3lb::MarchShape<float>::CY;
+  p.ntx = (d.sx + cx - 1) / cx;
+  p.nty = (d.sy + cy - 1) / cy;
+  const int64_t cols = int64_t(p.ntx) * p.nty;
+  double best = 0;
+  for (int k = 1; k <= d.sz; ++k) {
+    const double cost = double((cols * k + s->cus - 1) / s->cus) * ((d.sz + k - 1) / k + 2.5);
+    if (k == 1 || cost < best) {
+      best = cost;
+      p.nzc = k;
+    }
+  }
+  const double filled = double(d.np) / (best * s->cus * cx * cy);
+  p.on = s->march_test || filled >= (wide ? 0.5 : 0.65);
+  return p;
+}
+
+// Two steps from an even one.
+int launch_march(m3lb_solver* s, const m3lb::StepArgs& a, const MarchPlan& p) {
+  const m3lb::Dom& d = s->d;
+  m3lb::MarchArgs ma;
+  std::memset(&ma, 0, sizeof ma);
+  ma.a = a;
+  ma.a.remap = 32;  // the blocks an XCD holds at a time are neighbours in x, then y
+  for (int j = 0; j < 4; ++j) ma.a.macro[j] = nullptr;
+  ma.out = s->f_alt;
+  ma.ntx = p.ntx;
+  ma.nty = p.nty;
+  ma.nzc = p.nzc;
+  ma.core_y = d.sy / ma.nty;
+  ma.more_y = d.sy % ma.nty;
+  ma.run_z = d.sz / ma.nzc;
+  ma.more_z = d.sz % ma.nzc;
+  s->ks->march(ma, s->geometry || d.hx || d.hy || d.hz, s->stream);
+  std::swap(s->f, s->f_alt);
+  ++s->pair_passes;
+  return launch_ok();
+}
+
 }  // namespace
 
 extern "C" {
@@ -1017,6 +1083,13 @@ int m3lb_test_fail_fused_waits(m3lb_solver* s, int32_t on) {
   return M3LB_OK;
 }
 
+int m3lb_test_march_always(m3lb_solver* s, int32_t on) {
+  if (!s) return fail(M3LB_EINVAL, "null handle");
+  SYNC_OK(s);
+  s->march_test = on != 0;
+  return M3LB_OK;
+}
+
 int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   if (!s) return fail(M3LB_EINVAL, "null handle");
   if (nsteps < 0) return fail(M3LB_EINVAL, "nsteps must be >= 0");
@@ -1047,6 +1120,12 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   na.out = b.snap_d;
   for (int q = 0; q < 27; ++q) na.inv_scale[q] = s->inv_scale[q];
   const bool pairs = pair_eligible(s, a);
+  MarchPlan march = march_plan(s, a);
+  if (march.on && nsteps - int(s->t % 2) - (store_macroscopic ? 1 : 0) >= 2) {
+    const int rc = ensure_alt(s, s->geometry || s->d.hx || s->d.hy || s->d.hz);
+    if (rc) return rc;
+    if (s->alt_failed) march.on = false;
+  }
   PlanePlan plane = plane_plan(s);
   if (plane.steps && nsteps - int(s->t % 2) - (store_macroscopic ? 1 : 0) >= 2) {
     const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid);
@@ -1070,7 +1149,16 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
     }
     // two steps in one pass while two are left (never the step that stores
     // the macroscopic fields)
-    if (pairs && k + 1 < nsteps && !(store_macroscopic && k + 2 == nsteps)) {
+    if (march.on && left >= 2 && s->t % 2 == 0) {
+      const int rc = launch_march(s, a, march);
+      if (rc) return rc;
+      a.f = wa.f = sa.f = s->f;
+      na.f = s->f;
+      s->t += 2;
+      ++k;
+      continue;
+    }
+    if (pairs && !march.on && k + 1 < nsteps && !(store_macroscopic && k + 2 == nsteps)) {
       const int rc = launch_pair(s, a, int(s->t % 2));
       if (rc) return rc;
       s->t += 2;

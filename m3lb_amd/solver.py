@@ -73,6 +73,7 @@ SIGNATURES = {
     "m3lb_fused_passes": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_uint64)]),
     "m3lb_totals_static": (ctypes.c_int, [_vp, _dp]),
     "m3lb_test_fail_fused_waits": (ctypes.c_int, [_vp, ctypes.c_int32]),
+    "m3lb_test_march_always": (ctypes.c_int, [_vp, ctypes.c_int32]),
     "m3lb_initialize_taylor_green": (ctypes.c_int, [_vp, ctypes.c_double]),
     "m3lb_momentum_exchange": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_uint8), _dp]),
     # batched server
@@ -379,6 +380,10 @@ class FluidSolver:
     def test_fail_fused_waits(self, on):
         """m3lb_test_fail_fused_waits: failure-path test hook."""
         _check(self.L.m3lb_test_fail_fused_waits(self.h, 1 if on else 0))
+
+    def test_march_always(self, on):
+        """m3lb_test_march_always: test hook."""
+        _check(self.L.m3lb_test_march_always(self.h, 1 if on else 0))
 
     def set_tile_order(self, run):
         _check(self.L.m3lb_set_tile_order(self.h, int(run)))
