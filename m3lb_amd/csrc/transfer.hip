@@ -20,6 +20,7 @@ int err(int code, const std::string& m) { return set_error(code, m.c_str()); }
 
 struct Slot {
   int device = -1;
+  size_t bytes = 0;
   void* host = nullptr;  // pinned, written and read by the device in place
   hipEvent_t done = nullptr;
 };
@@ -38,15 +39,16 @@ class Pool {
     free_.clear();
     total_ = 0;
   }
-  // Up to `want` slots of `device`; at least one, waiting while other calls
-  // hold them all.  Empty with *rc set when not even one can be had.
-  std::vector<Slot> take(int device, int want, int* rc) {
+  // Up to `want` slots of `device` and at least `bytes`; at least one, waiting
+  // while other calls hold them all.  Empty with *rc set when not even one can be
+  // had.
+  std::vector<Slot> take(int device, int want, size_t bytes, int* rc) {
     std::unique_lock<std::mutex> l(mu_);
     std::vector<Slot> got;
     *rc = M3LB_OK;
     for (;;) {
       for (size_t k = 0; k < free_.size() && int(got.size()) < want;) {
-        if (free_[k].device == device) {
+        if (free_[k].device == device && free_[k].bytes >= bytes) {
           got.push_back(free_[k]);
           free_.erase(free_.begin() + std::ptrdiff_t(k));
         } else {
@@ -55,12 +57,12 @@ class Pool {
       }
       while (int(got.size()) < want && total_ < kSlots) {
         Slot s;
-        if (!make(device, s)) break;
+        if (!make(device, bytes, s)) break;
         ++total_;
         got.push_back(s);
       }
       if (!got.empty()) return got;
-      if (!free_.empty()) {  // all free ones belong to another device
+      if (!free_.empty()) {  // all free ones are too small or another device's
         drop(free_.back());
         free_.pop_back();
         --total_;
@@ -82,12 +84,13 @@ class Pool {
   }
 
  private:
-  static bool make(int device, Slot& s) {
+  static bool make(int device, size_t bytes, Slot& s) {
     int cur = device;
     (void)hipGetDevice(&cur);
     if (cur != device && hipSetDevice(device) != hipSuccess) return false;
     s.device = device;
-    bool ok = hipHostMalloc(&s.host, kSlotBytes, hipHostMallocDefault) == hipSuccess;
+    s.bytes = bytes;
+    bool ok = hipHostMalloc(&s.host, bytes, hipHostMallocDefault) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
       (void)hipGetLastError();
@@ -122,13 +125,16 @@ int cpus() {
 
 // Runs fn(chunk, slot) for every chunk, each thread with a slot of its own;
 // the caller is one of the threads.  fn returns an M3LB code; the first
-// failure stops the rest.
+// failure stops the rest.  `bytes` is what one chunk takes: pinning a whole slot
+// is 0.1 ms, which a program of small boxes would notice, so a call that
+// needs less than a small slot asks for no more.
 template <class Fn>
-int each_chunk(size_t chunks, int device, Fn&& fn) {
+int each_chunk(size_t chunks, size_t bytes, int device, Fn&& fn) {
   if (chunks == 0) return M3LB_OK;
   static const int most = std::max(1, std::min(kSlots - 4, cpus() - 2));
   int rc = M3LB_OK;
-  std::vector<Slot> slots = pool().take(device, int(std::min<size_t>(chunks, size_t(most))), &rc);
+  std::vector<Slot> slots = pool().take(device, int(std::min<size_t>(chunks, size_t(most))),
+                                       bytes <= kSmallSlotBytes ? kSmallSlotBytes : kSlotBytes, &rc);
   if (rc) return err(rc, "pinned staging memory");
   std::atomic<size_t> next{0};
   std::atomic<int> first_rc{M3LB_OK};
@@ -200,8 +206,8 @@ int read_macroscopic(const KernelSet* ks, ReadArgs a, int device, hipStream_t st
                      double* const dst[4]) {
   const size_t np = size_t(a.d.np), rb = size_t(ks->real_bytes);
   // whole multiples of 64 nodes, so that every plane of a slot starts aligned
-  const size_t per = kSlotBytes / (4 * rb) / 64 * 64;
-  return each_chunk((np + per - 1) / per, device, [&](size_t c, const Slot& s) -> int {
+  const size_t per = std::min(kSlotBytes / (4 * rb) / 64 * 64, (np + 63) / 64 * 64);
+  return each_chunk((np + per - 1) / per, per * 4 * rb, device, [&](size_t c, const Slot& s) -> int {
     ReadArgs r = a;
     r.n0 = int(c * per);
     r.n1 = int(std::min(np, (c + 1) * per));
@@ -222,7 +228,7 @@ int read_populations(const KernelSet* ks, ReadArgs a, int q, bool logical, int d
                      hipStream_t st, double* dst) {
   const size_t np = size_t(a.d.np), rb = size_t(ks->real_bytes), row = size_t(q);
   const size_t per = kSlotBytes / (row * rb) / kBlock * kBlock;
-  return each_chunk((np + per - 1) / per, device, [&](size_t c, const Slot& s) -> int {
+  return each_chunk((np + per - 1) / per, std::min(np, per) * row * rb, device, [&](size_t c, const Slot& s) -> int {
     ReadArgs r = a;
     r.n0 = int(c * per);
     r.n1 = int(std::min(np, (c + 1) * per));
@@ -239,7 +245,7 @@ int read_populations(const KernelSet* ks, ReadArgs a, int q, bool logical, int d
 
 int upload_real(void* dst, const double* src, size_t n, int real_bytes, int device, hipStream_t st) {
   const size_t rb = size_t(real_bytes), per = kSlotBytes / rb;
-  return each_chunk((n + per - 1) / per, device, [&](size_t c, const Slot& s) -> int {
+  return each_chunk((n + per - 1) / per, std::min(n, per) * rb, device, [&](size_t c, const Slot& s) -> int {
     const size_t k0 = c * per, k1 = std::min(n, k0 + per);
     if (real_bytes == 8) {
       std::memcpy(s.host, src + k0, (k1 - k0) * rb);
@@ -255,7 +261,7 @@ int upload_real(void* dst, const double* src, size_t n, int real_bytes, int devi
 }
 
 int upload_bytes(void* dst, const void* src, size_t n, int device, hipStream_t st) {
-  return each_chunk((n + kSlotBytes - 1) / kSlotBytes, device, [&](size_t c, const Slot& s) -> int {
+  return each_chunk((n + kSlotBytes - 1) / kSlotBytes, std::min(n, kSlotBytes), device, [&](size_t c, const Slot& s) -> int {
     const size_t k0 = c * kSlotBytes, m = std::min(n - k0, kSlotBytes);
     std::memcpy(s.host, static_cast<const char*>(src) + k0, m);
     if (hipMemcpyAsync(static_cast<char*>(dst) + k0, s.host, m, hipMemcpyHostToDevice, st) !=
@@ -269,7 +275,7 @@ int read_column_sums(const double* partial_d, unsigned grid, int cols, int devic
                      double* out) {
   const size_t bytes = size_t(grid) * size_t(cols) * sizeof(double);
   if (bytes > kSlotBytes) return err(M3LB_EINVAL, "too many reduction partials");
-  return each_chunk(1, device, [&](size_t, const Slot& s) -> int {
+  return each_chunk(1, bytes, device, [&](size_t, const Slot& s) -> int {
     if (hipMemcpyAsync(s.host, partial_d, bytes, hipMemcpyDeviceToHost, st) != hipSuccess)
       return err(M3LB_EDEVICE, "partials download failed");
     const int rc = wait_for(s, st);

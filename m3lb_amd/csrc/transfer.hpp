@@ -26,6 +26,7 @@ namespace m3lb {
 // other beyond that), allocated when first needed and given back when the last
 // handle is destroyed.
 constexpr size_t kSlotBytes = 4u << 20;
+constexpr size_t kSmallSlotBytes = 512u << 10;
 constexpr int kSlots = 16;
 
 // One reference per live solver or server.
