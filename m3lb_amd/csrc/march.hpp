@@ -41,6 +41,7 @@
 #pragma once
 
 #include "kernels.hpp"
+#include "wrap.hpp"
 
 namespace m3lb {
 
@@ -106,7 +107,7 @@ __global__ void __launch_bounds__(MarchShape<typename K::T>::NT) k_march(MarchAr
   const bool own_r = cx >= 1 && cx < nx + 1, own_l = cx >= 3 && cx < nx + 3;  // x + 1, x - 1
   bool in = c < NP && cx <= nx + 3 && cy <= ny + 1;  // takes part in A
   int X = X0 - 2 + cx, Y = Y0 - 1 + cy;
-  if (d.px) X = int(unsigned(X + 2 * d.sx) % unsigned(d.sx));  // X >= -2
+  if (d.px) X = wrapped(X, d.sx);
   auto wrap = [](int& v, int n, bool per) -> bool {  // v in -1 .. n, false: outside
     if (v >= 0 && v < n) return true;
     v = v < 0 ? v + n : v - n;

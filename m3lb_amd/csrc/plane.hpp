@@ -26,6 +26,7 @@
 #pragma once
 
 #include "kernels.hpp"
+#include "wrap.hpp"
 
 namespace m3lb {
 
@@ -168,11 +169,11 @@ __global__ void __launch_bounds__(S::NT) k_plane(PlaneArgs pa) {
     Y = Y0 - H + c / RX;
     if (X < 0 || X >= d.sx) {
       if (!d.px) return false;
-      X = int(unsigned(X + d.sx * H) % unsigned(d.sx));  // X >= -H
+      X = wrapped(X, d.sx);
     }
     if (Y < 0 || Y >= d.sy) {
       if (!d.py) return false;
-      Y = int(unsigned(Y + d.sy * H) % unsigned(d.sy));
+      Y = wrapped(Y, d.sy);
     }
     return true;
   };
