@@ -980,8 +980,9 @@ int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& 
   pa.core_y = s->d.sy / pa.nty;
   pa.more_y = s->d.sy % pa.nty;
   s->ks->plane(pa, p.shape, p.nodes, s->stream);
-  std::swap(s->f, s->f_alt);
-  return launch_ok();
+  const int rc = launch_ok();
+  if (!rc) std::swap(s->f, s->f_alt);  // a refused launch leaves the box as it was
+  return rc;
 }
 
 // Two steps per pass through LDS (march.hpp).  The blocks along z are chosen for
@@ -1043,9 +1044,11 @@ int launch_march(m3lb_solver* s, const m3lb::StepArgs& a, const MarchPlan& p) {
   ma.run_z = d.sz / ma.nzc;
   ma.more_z = d.sz % ma.nzc;
   s->ks->march(ma, s->geometry || d.hx || d.hy || d.hz, s->stream);
+  const int rc = launch_ok();
+  if (rc) return rc;  // a refused launch leaves the box as it was
   std::swap(s->f, s->f_alt);
   ++s->pair_passes;
-  return launch_ok();
+  return M3LB_OK;
 }
 
 }  // namespace
@@ -1094,6 +1097,7 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   if (!s) return fail(M3LB_EINVAL, "null handle");
   if (nsteps < 0) return fail(M3LB_EINVAL, "nsteps must be >= 0");
   if (nsteps == 0) return M3LB_OK;
+  s->macro_valid = false;  // also if a later pass of this call fails
   m3lb::StepArgs a = step_args(s);
   if (store_macroscopic) {
     for (int k = 0; k < 4; ++k) {
