@@ -82,6 +82,14 @@ class Pool {
     }
     cv_.notify_all();
   }
+  // Slots that the device may still write, for good: not used again and not freed.
+  void forget(size_t n) {
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      total_ -= int(n);
+    }
+    cv_.notify_all();
+  }
 
  private:
   static bool make(int device, size_t bytes, Slot& s) {
@@ -125,11 +133,13 @@ int cpus() {
 
 // Runs fn(chunk, slot) for every chunk, each thread with a slot of its own;
 // the caller is one of the threads.  fn returns an M3LB code; the first
-// failure stops the rest.  `bytes` is what one chunk takes: pinning a whole slot
+// failure stops the rest.  After a failure work that fn queued on `st` may still
+// read or write a slot, so the slots go back only once the stream has been waited
+// for.  `bytes` is what one chunk takes: pinning a whole slot
 // is 0.1 ms, which a program of small boxes would notice, so a call that
 // needs less than a small slot asks for no more.
 template <class Fn>
-int each_chunk(size_t chunks, size_t bytes, int device, Fn&& fn) {
+int each_chunk(size_t chunks, size_t bytes, int device, hipStream_t st, Fn&& fn) {
   if (chunks == 0) return M3LB_OK;
   static const int most = std::max(1, std::min(kSlots - 4, cpus() - 2));
   int rc = M3LB_OK;
@@ -170,7 +180,8 @@ int each_chunk(size_t chunks, size_t bytes, int device, Fn&& fn) {
   }
   body(slots[0], false);
   for (std::thread& t : threads) t.join();
-  pool().give(slots);
+  if (first_rc.load() == M3LB_OK || hipStreamSynchronize(st) == hipSuccess) pool().give(slots);
+  else pool().forget(slots.size());
   if (first_rc.load()) return err(first_rc.load(), msg.empty() ? "staged transfer failed" : msg);
   return M3LB_OK;
 }
@@ -207,7 +218,7 @@ int read_macroscopic(const KernelSet* ks, ReadArgs a, int device, hipStream_t st
   const size_t np = size_t(a.d.np), rb = size_t(ks->real_bytes);
   // whole multiples of 64 nodes, so that every plane of a slot starts aligned
   const size_t per = std::min(kSlotBytes / (4 * rb) / 64 * 64, (np + 63) / 64 * 64);
-  return each_chunk((np + per - 1) / per, per * 4 * rb, device, [&](size_t c, const Slot& s) -> int {
+  return each_chunk((np + per - 1) / per, per * 4 * rb, device, st, [&](size_t c, const Slot& s) -> int {
     ReadArgs r = a;
     r.n0 = int(c * per);
     r.n1 = int(std::min(np, (c + 1) * per));
@@ -228,7 +239,7 @@ int read_populations(const KernelSet* ks, ReadArgs a, int q, bool logical, int d
                      hipStream_t st, double* dst) {
   const size_t np = size_t(a.d.np), rb = size_t(ks->real_bytes), row = size_t(q);
   const size_t per = kSlotBytes / (row * rb) / kBlock * kBlock;
-  return each_chunk((np + per - 1) / per, std::min(np, per) * row * rb, device, [&](size_t c, const Slot& s) -> int {
+  return each_chunk((np + per - 1) / per, std::min(np, per) * row * rb, device, st, [&](size_t c, const Slot& s) -> int {
     ReadArgs r = a;
     r.n0 = int(c * per);
     r.n1 = int(std::min(np, (c + 1) * per));
@@ -245,7 +256,7 @@ int read_populations(const KernelSet* ks, ReadArgs a, int q, bool logical, int d
 
 int upload_real(void* dst, const double* src, size_t n, int real_bytes, int device, hipStream_t st) {
   const size_t rb = size_t(real_bytes), per = kSlotBytes / rb;
-  return each_chunk((n + per - 1) / per, std::min(n, per) * rb, device, [&](size_t c, const Slot& s) -> int {
+  return each_chunk((n + per - 1) / per, std::min(n, per) * rb, device, st, [&](size_t c, const Slot& s) -> int {
     const size_t k0 = c * per, k1 = std::min(n, k0 + per);
     if (real_bytes == 8) {
       std::memcpy(s.host, src + k0, (k1 - k0) * rb);
@@ -261,7 +272,7 @@ int upload_real(void* dst, const double* src, size_t n, int real_bytes, int devi
 }
 
 int upload_bytes(void* dst, const void* src, size_t n, int device, hipStream_t st) {
-  return each_chunk((n + kSlotBytes - 1) / kSlotBytes, std::min(n, kSlotBytes), device, [&](size_t c, const Slot& s) -> int {
+  return each_chunk((n + kSlotBytes - 1) / kSlotBytes, std::min(n, kSlotBytes), device, st, [&](size_t c, const Slot& s) -> int {
     const size_t k0 = c * kSlotBytes, m = std::min(n - k0, kSlotBytes);
     std::memcpy(s.host, static_cast<const char*>(src) + k0, m);
     if (hipMemcpyAsync(static_cast<char*>(dst) + k0, s.host, m, hipMemcpyHostToDevice, st) !=
@@ -275,7 +286,7 @@ int read_column_sums(const double* partial_d, unsigned grid, int cols, int devic
                      double* out) {
   const size_t bytes = size_t(grid) * size_t(cols) * sizeof(double);
   if (bytes > kSlotBytes) return err(M3LB_EINVAL, "too many reduction partials");
-  return each_chunk(1, bytes, device, [&](size_t, const Slot& s) -> int {
+  return each_chunk(1, bytes, device, st, [&](size_t, const Slot& s) -> int {
     if (hipMemcpyAsync(s.host, partial_d, bytes, hipMemcpyDeviceToHost, st) != hipSuccess)
       return err(M3LB_EDEVICE, "partials download failed");
     const int rc = wait_for(s, st);
