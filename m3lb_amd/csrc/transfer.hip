@@ -98,7 +98,10 @@ class Pool {
     if (cur != device && hipSetDevice(device) != hipSuccess) return false;
     s.device = device;
     s.bytes = bytes;
-    bool ok = hipHostMalloc(&s.host, bytes, hipHostMallocDefault) == hipSuccess;
+    // The host reads a slot after a wait for this event alone, which need not
+    // release to the system: so the memory is coherent by itself, whatever the
+    // process's default is.  (An event that releases costs 1 us a readout.)
+    bool ok = hipHostMalloc(&s.host, bytes, hipHostMallocCoherent) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
       (void)hipGetLastError();

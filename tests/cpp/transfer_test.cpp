@@ -21,7 +21,7 @@ std::set<char*> g_in_flight;            // pinned ranges that the device may sti
 std::map<hipEvent_t, char*> g_event_of; // what the event's last record waits for
 thread_local char* t_last = nullptr;    // range of this thread's last launch
 std::atomic<int> g_fail_records{0}, g_fail_syncs{0}, g_fail_mallocs{0};
-std::atomic<int> g_peak{0}, g_mallocs{0}, g_reused{0};
+std::atomic<int> g_peak{0}, g_mallocs{0}, g_incoherent{0}, g_device_events{0}, g_reused{0};
 thread_local std::string t_msg;
 
 char* range_of(const void* p) {
@@ -52,12 +52,13 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipExtGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "failed by the test"; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
   if (g_fail_mallocs > 0) { --g_fail_mallocs; return hipErrorOutOfMemory; }
   *p = std::malloc(n);
   std::lock_guard<std::mutex> l(g_mu);
   g_pinned[static_cast<char*>(*p)] = n;
   ++g_mallocs;
+  if (!(flags & hipHostMallocCoherent)) ++g_incoherent;
   if (int(g_pinned.size()) > g_peak) g_peak = int(g_pinned.size());
   return hipSuccess;
 }
@@ -68,7 +69,8 @@ hipError_t hipHostFree(void* p) {
   std::free(p);
   return hipSuccess;
 }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned flags) {
+  if (!(flags & hipEventReleaseToSystem)) ++g_device_events;
   *e = reinterpret_cast<hipEvent_t>(std::malloc(1));
   return hipSuccess;
 }
@@ -165,7 +167,12 @@ int upload(size_t n) {
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   m3lb::staging_acquire();
-  if (what == "failed_wait") {
+  if (what == "visible") {
+    REQUIRE(fields(100) == M3LB_OK && fields(1500000) == M3LB_OK);
+    // the host sees what kernels wrote after the wait: coherent memory, or events
+    // that release to the system
+    REQUIRE(g_incoherent == 0 || g_device_events == 0);
+  } else if (what == "failed_wait") {
     // one wait of several fails: none of the slots is used again before the work
     // in flight has ended
     for (int np : {100, 1500000}) {

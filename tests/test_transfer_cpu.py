@@ -1,7 +1,8 @@
 """CPU test of the staged transfers (m3lb_amd/csrc/transfer.hip) with the runtime's
-entry points stood in for (tests/cpp/transfer_test.cpp): slots of a failed call are
-not handed on while the device may write them, calls of several threads share at
-most kSlots slots, and running out of pinned memory is an error, not a hang."""
+entry points stood in for (tests/cpp/transfer_test.cpp): what the host reads after a
+wait is visible to it, slots of a failed call are not handed on while the device
+may write them, calls of several threads share at most kSlots slots, and running
+out of pinned memory is an error, not a hang."""
 import os
 import subprocess
 
@@ -27,7 +28,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["failed_wait", "threads", "no_memory"])
+@pytest.mark.parametrize("case", ["visible", "failed_wait", "threads", "no_memory"])
 def test_staged_transfers(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
