@@ -1125,13 +1125,21 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   for (int q = 0; q < 27; ++q) na.inv_scale[q] = s->inv_scale[q];
   const bool pairs = pair_eligible(s, a);
   MarchPlan march = march_plan(s, a);
-  if (march.on && nsteps - int(s->t % 2) - (store_macroscopic ? 1 : 0) >= 2) {
+  // An even number of steps from an odd one costs the passes through LDS two single
+  // steps, the passes in place none.  us per step, in place / single steps and
+  // LDS, D3Q27 CM: FP32 512^3 2 steps 4176 / 5341, 6 4180 / 4372, 8 4180 / 4234, 10
+  // 4180 / 4154, 20 4182 / 3992; 256^3 2 558 / 667, 8 550 / 549; FP64 256^3 2 1098 /
+  // 1384, 8 1087 / 1143, 10 1085 / 1119, 20 1079 / 1075 (on a card with 1295 in place
+  // 20 1086).
+  const int passable = nsteps - (store_macroscopic ? 1 : 0);
+  if (march.on && pairs && s->t % 2 == 1 && passable % 2 == 0 && passable < 10) march.on = false;
+  if (march.on && passable - int(s->t % 2) >= 2) {
     const int rc = ensure_alt(s, s->geometry || s->d.hx || s->d.hy || s->d.hz);
     if (rc) return rc;
     if (s->alt_failed) march.on = false;
   }
   PlanePlan plane = plane_plan(s);
-  if (plane.steps && nsteps - int(s->t % 2) - (store_macroscopic ? 1 : 0) >= 2) {
+  if (plane.steps && passable - int(s->t % 2) >= 2) {
     const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid);
     if (rc) return rc;
     if (s->alt_failed) plane.steps = 0;
