@@ -10,6 +10,7 @@
 #include "march.hpp"
 #include "pair.hpp"
 #include "plane.hpp"
+#include "step_plan.hpp"
 
 namespace m3lb {
 
@@ -47,13 +48,16 @@ struct KernelSet {
   void (*march)(const MarchArgs&, bool geom, hipStream_t);
 };
 
-// Regions of the plane kernel (PlaneArgs) and what moves in the box.
-enum PlaneRegion { kPlaneSquare = 0, kPlaneWide = 1, kPlaneSmall = 2 };
-enum PlaneNodes { kPlaneFluid = 0, kPlaneGeom = 1, kPlaneWalls = 2 };
-using PlaneSquare = PlaneShape<32, 32, 1024>;
-using PlaneWide = PlaneShape<64, 32, 512>;
-using PlaneSmall = PlaneShape<24, 24, 576>;
-using PlaneWalled = PlaneShape<32, 28, 896, true>;
+// Shapes of the plane kernel, by the regions of its plan.
+template <int SHAPE, int NODES, int NF, bool WAVES = false>
+using PlaneOf = PlaneShape<plane_region(SHAPE, NODES).x, plane_region(SHAPE, NODES).y, NF, WAVES>;
+using PlaneSquare = PlaneOf<kPlaneSquare, kPlaneFluid, 1024>;
+using PlaneWide = PlaneOf<kPlaneWide, kPlaneFluid, 512>;
+using PlaneSmall = PlaneOf<kPlaneSmall, kPlaneFluid, 576>;
+using PlaneWalled = PlaneOf<kPlaneSquare, kPlaneWalls, 896, true>;
+static_assert(MarchShape<double>::W == march_core(8).x && MarchShape<double>::CY == march_core(8).y &&
+                  MarchShape<float>::W == march_core(4).x && MarchShape<float>::CY == march_core(4).y,
+              "the plan's cores are the kernel's");
 
 inline unsigned blocks_for(long long n) { return unsigned((n + kBlock - 1) / kBlock); }
 

@@ -864,76 +864,23 @@ int launch_pair(m3lb_solver* s, const m3lb::StepArgs& a, int parity) {
 // Several steps of a plane box per launch (plane.hpp).  Applies to a box whose
 // moving nodes read no other node's set (no outlets, no specular cells, corner
 // stencils on walls) and unless fusion is off.
-struct PlanePlan {
-  int steps = 0;  // most steps per launch, even; 0: one launch per step
-  int shape = 0, nodes = 0;
-};
-
-int plane_margin(int steps, int nodes) { return steps + (nodes == m3lb::kPlaneWalls ? 2 : 0); }
-struct PlaneRegionSize {
-  int x, y;
-};
-PlaneRegionSize region_size(int shape, int nodes) {
-  using namespace m3lb;
-  if (nodes == kPlaneWalls) return {PlaneWalled::RX, PlaneWalled::RY};
-  if (shape == kPlaneSmall) return {PlaneSmall::RX, PlaneSmall::RY};
-  if (shape == kPlaneWide) return {PlaneWide::RX, PlaneWide::RY};
-  return {PlaneSquare::RX, PlaneSquare::RY};
-}
-
-// Region and steps per launch.  While the blocks of a region fit the chip in
-// one round, a launch lasts as long as one block: the most steps that still
-// fit, in the smallest region (fewer nodes of margin per wave).  us per step,
-// FP64 BGK / FP32 CM:
-//   128^2  24 x 24 regions, 8 steps 1.17 / 1.05; 32 x 32, 8 1.34 / 1.21
-//   192^2  24 x 24, 6 1.42 / 1.24;  32 x 32, 8 1.50 / 1.32
-//   256^2  32 x 32, 8 1.67 / 1.41;  6 steps 1.80 / 1.56
-//   320^2  32 x 32, 6 1.95 / 1.63;  8 steps (two rounds) 2.76 / 2.16
-//   384^2  32 x 32, 4 2.41 / 2.09;  6 steps 2.98 / 2.47, 8 3.67 / 2.95
-// with walls (cavity FP64 CM): 129^2 8 steps 3.7, 6 3.8, 4 4.5; 257^2 4.7, 5.6, 7.8.
-// Larger planes are bound by traffic and by the work on margins: 4-byte and
-// 2-byte populations take 64 x 32 regions and 6 steps (1024^2 FP32 7.9 us per
-// step, 8.0 at 4 steps, 9.3 with 32 x 32 regions, 11.1 one launch per step;
-// 4096^2 93, 96, 125 and 189), 8-byte ones 32 x 32 and 4 (1024^2 12.0 us, 12.2
-// at 6, 13.5 with 64 x 32 regions, 23.6 one launch per step; 4096^2 169 and 426).
-PlanePlan plane_plan(const m3lb_solver* s) {
-  PlanePlan p;
+m3lb::PlanePlan plane_plan(const m3lb_solver* s) {
   const Boundaries& b = s->b;
   const m3lb::Dom& d = s->d;
-  if (!s->ks->plane || s->fusion == M3LB_FUSION_OFF || s->alt_failed || s->Q != 9) return p;
-  if (b.nspec || b.nsnap || (b.nwall && !b.local)) return p;
+  if (!s->ks->plane || s->fusion == M3LB_FUSION_OFF || s->alt_failed || s->Q != 9) return {};
+  if (b.nspec || b.nsnap || (b.nwall && !b.local)) return {};
   // an unwrapped axis without a halo (one node, not periodic) has no margin
-  if (!(d.px || d.hx) || !(d.py || d.hy)) return p;
+  if (!(d.px || d.hx) || !(d.py || d.hy)) return {};
+  m3lb::PlaneBox p;
+  p.sx = d.sx;
+  p.sy = d.sy;
   p.nodes = b.nwall ? m3lb::kPlaneWalls
                     : (s->geometry || d.hx || d.hy ? m3lb::kPlaneGeom : m3lb::kPlaneFluid);
-  const int steps_shapes[5][2] = {{8, m3lb::kPlaneSmall},  {6, m3lb::kPlaneSmall},
-                                  {8, m3lb::kPlaneSquare}, {6, m3lb::kPlaneSquare},
-                                  {4, m3lb::kPlaneSquare}};
-  for (const auto& c : steps_shapes) {
-    if (b.nwall && c[1] == m3lb::kPlaneSmall) continue;
-    const PlaneRegionSize r = region_size(c[1], p.nodes);
-    const int h = plane_margin(c[0], p.nodes), cx = r.x - 2 * h, cy = r.y - 2 * h;
-    if (int64_t((d.sx + cx - 1) / cx) * ((d.sy + cy - 1) / cy) > s->cus) continue;
-    p.steps = c[0];
-    p.shape = c[1];
-    return p;
-  }
-  p.shape = m3lb::kPlaneSquare;
-  if (b.nwall || s->ks->elem_bytes == 8) {
-    p.steps = 4;
-  } else {
-    p.shape = m3lb::kPlaneWide;
-    p.steps = 6;
-    // 2-byte populations beyond the caches' reach of one XCD gain little (D2Q9
-    // CM 2048^2, us per step: FP16 27.2 against 27.3, BF16 25.7 / 28.1, I16
-    // 24.7 / 28.5), and E2M13 (32.0 / 30.6, its codec runs on the margins too)
-    // and boxes with geometry (FP16 28.2 / 27.6, E2M13 34.0 / 29.4) lose
-    const uint64_t bytes = s->stride * uint64_t(s->Q) * uint64_t(s->ks->elem_bytes);
-    if (s->ks->elem_bytes == 2 && bytes > (32u << 20) &&
-        (s->cfg.dtype == M3LB_E2M13 || p.nodes == m3lb::kPlaneGeom))
-      p.steps = 0;
-  }
-  return p;
+  p.elem_bytes = s->ks->elem_bytes;
+  p.e2m13 = s->cfg.dtype == M3LB_E2M13;
+  p.bytes = s->stride * uint64_t(s->Q) * uint64_t(s->ks->elem_bytes);
+  p.cus = s->cus;
+  return m3lb::plane_rule(p);
 }
 
 // The second population array: allocated at the first pass, and given the
@@ -961,7 +908,7 @@ int ensure_alt(m3lb_solver* s, bool statics) {
 
 // `steps` (even) steps from an even one.
 int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& wa,
-                 const PlanePlan& p, int steps) {
+                 const m3lb::PlanePlan& p, int steps) {
   m3lb::PlaneArgs pa;
   std::memset(&pa, 0, sizeof pa);
   pa.a = a;
@@ -970,11 +917,10 @@ int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& 
   pa.w = wa;
   pa.out = s->f_alt;
   pa.steps = steps;
-  pa.margin = plane_margin(steps, p.nodes);
-  const PlaneRegionSize r = region_size(p.shape, p.nodes);
-  const int cx = r.x - 2 * pa.margin, cy = r.y - 2 * pa.margin;
-  pa.ntx = (s->d.sx + cx - 1) / cx;
-  pa.nty = (s->d.sy + cy - 1) / cy;
+  pa.margin = m3lb::plane_margin(steps, p.nodes);
+  const m3lb::PlaneGrid g = m3lb::plane_grid(s->d.sx, s->d.sy, steps, p.shape, p.nodes);
+  pa.ntx = g.ntx;
+  pa.nty = g.nty;
   pa.core_x = s->d.sx / pa.ntx;
   pa.more_x = s->d.sx % pa.ntx;
   pa.core_y = s->d.sy / pa.nty;
@@ -985,50 +931,27 @@ int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& 
   return rc;
 }
 
-// Two steps per pass through LDS (march.hpp).  The blocks along z are chosen for
-// the least rounds of blocks times planes of one (two planes and about half a
-// plane's time of start are extra).  It applies beyond the caches (within them a
-// step is bound by its arithmetic and loses to the margins: D3Q27 CM FP32 128^3
-// 28.1 GLUPS against 30.8) and where that schedule keeps the chip's cells filled:
-// 4-byte storage gains from 0.76 on (192^3 35.5 against 29.6 for the pass of
-// pair.hpp; 0.62, 160^3: 28.3 against 28.9), 8-byte from 0.55 (150x130x140 16.1
-// against 13.0).  It needs a second population array; where there is no room for
-// one, or the caller set the tuning values of pair.hpp, that pass runs.
-struct MarchPlan {
-  bool on = false;
-  int ntx = 0, nty = 0, nzc = 0;
-};
-MarchPlan march_plan(const m3lb_solver* s, const m3lb::StepArgs& a) {
-  MarchPlan p;
+// Two steps per pass through LDS (march.hpp).  Applies beyond the caches (within them
+// a step is bound by its arithmetic and loses to the margins: D3Q27 CM FP32 128^3
+// 28.1 GLUPS against 30.8) and where its blocks fill the chip.  It needs a second
+// population array; where there is no room for one, or the caller set the tuning
+// values of pair.hpp, that pass runs.
+m3lb::MarchPlan march_plan(const m3lb_solver* s, const m3lb::StepArgs& a) {
   const m3lb::Dom& d = s->d;
-  if (!s->ks->march || s->fusion != M3LB_FUSION_AUTO || s->alt_failed) return p;
-  if (s->b.nwall || s->b.nspec || s->b.nsnap) return p;
+  if (!s->ks->march || s->fusion != M3LB_FUSION_AUTO || s->alt_failed) return {};
+  if (s->b.nwall || s->b.nspec || s->b.nsnap) return {};
   if (!s->march_test &&
       (a.cached || s->pair_stripes || s->pair_lag || s->pair_bpc || s->pair_group))
-    return p;
+    return {};
   // an unwrapped axis without a halo (one node, not periodic) has no margin
-  if (!(d.px || d.hx) || !(d.py || d.hy) || !(d.pz || d.hz)) return p;
-  const bool wide = s->ks->elem_bytes == 8;
-  const int cx = wide ? m3lb::MarchShape<double>::W : m3lb::MarchShape<float>::W;
-  const int cy = wide ? m3lb::MarchShape<double>::CY : m3lb::MarchShape<float>::CY;
-  p.ntx = (d.sx + cx - 1) / cx;
-  p.nty = (d.sy + cy - 1) / cy;
-  const int64_t cols = int64_t(p.ntx) * p.nty;
-  double best = 0;
-  for (int k = 1; k <= d.sz; ++k) {
-    const double cost = double((cols * k + s->cus - 1) / s->cus) * ((d.sz + k - 1) / k + 2.5);
-    if (k == 1 || cost < best) {
-      best = cost;
-      p.nzc = k;
-    }
-  }
-  const double filled = double(d.np) / (best * s->cus * cx * cy);
-  p.on = s->march_test || filled >= (wide ? 0.5 : 0.65);
+  if (!(d.px || d.hx) || !(d.py || d.hy) || !(d.pz || d.hz)) return {};
+  m3lb::MarchPlan p = m3lb::march_rule({d.sx, d.sy, d.sz, s->ks->elem_bytes, s->cus});
+  p.on = p.on || s->march_test;
   return p;
 }
 
 // Two steps from an even one.
-int launch_march(m3lb_solver* s, const m3lb::StepArgs& a, const MarchPlan& p) {
+int launch_march(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::MarchPlan& p) {
   const m3lb::Dom& d = s->d;
   m3lb::MarchArgs ma;
   std::memset(&ma, 0, sizeof ma);
@@ -1124,7 +1047,7 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   na.out = b.snap_d;
   for (int q = 0; q < 27; ++q) na.inv_scale[q] = s->inv_scale[q];
   const bool pairs = pair_eligible(s, a);
-  MarchPlan march = march_plan(s, a);
+  m3lb::MarchPlan march = march_plan(s, a);
   // An even number of steps from an odd one costs the passes through LDS two single
   // steps, the passes in place none.  us per step, in place / single steps and
   // LDS, D3Q27 CM: FP32 512^3 2 steps 4176 / 5341, 6 4180 / 4372, 8 4180 / 4234, 10
@@ -1138,7 +1061,7 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
     if (rc) return rc;
     if (s->alt_failed) march.on = false;
   }
-  PlanePlan plane = plane_plan(s);
+  m3lb::PlanePlan plane = plane_plan(s);
   if (plane.steps && passable - int(s->t % 2) >= 2) {
     const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid);
     if (rc) return rc;

@@ -1,0 +1,140 @@
+// step_plan.hpp -- which pass takes the steps of a box, and in what blocks: the
+// rules of the D2Q9 passes (plane.hpp) and of the D3Q27 passes through LDS
+// (march.hpp).  Plain C++ without HIP, so that the CPU tests can check them
+// (tests/cpp/step_plan_test.cpp).
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+namespace m3lb {
+
+// ---- several D2Q9 steps per launch ----
+// Regions of the plane kernel and what moves in the box.
+enum PlaneRegion { kPlaneSquare = 0, kPlaneWide = 1, kPlaneSmall = 2 };
+enum PlaneNodes { kPlaneFluid = 0, kPlaneGeom = 1, kPlaneWalls = 2 };
+
+struct RegionSize {
+  int x, y;
+};
+constexpr RegionSize plane_region(int shape, int nodes) {
+  return nodes == kPlaneWalls    ? RegionSize{32, 28}
+         : shape == kPlaneSmall  ? RegionSize{24, 24}
+         : shape == kPlaneWide   ? RegionSize{64, 32}
+                                 : RegionSize{32, 32};
+}
+
+// With walls a corner sees two nodes further than a fluid node does.
+constexpr int plane_margin(int steps, int nodes) { return steps + (nodes == kPlaneWalls ? 2 : 0); }
+
+// Blocks of a pass of `steps` steps along each axis.
+struct PlaneGrid {
+  int ntx, nty;
+};
+inline PlaneGrid plane_grid(int sx, int sy, int steps, int shape, int nodes) {
+  const RegionSize r = plane_region(shape, nodes);
+  const int h = plane_margin(steps, nodes), cx = r.x - 2 * h, cy = r.y - 2 * h;
+  return {(sx + cx - 1) / cx, (sy + cy - 1) / cy};
+}
+
+struct PlaneBox {
+  int sx, sy;      // padded extents
+  int nodes;       // PlaneNodes
+  int elem_bytes;  // per stored population
+  bool e2m13;
+  uint64_t bytes;  // of the population array
+  int cus;
+};
+
+struct PlanePlan {
+  int steps = 0;  // most steps per launch, even; 0: one launch per step
+  int shape = 0, nodes = 0;
+};
+
+// Region and steps per launch.  While the blocks of a region fit the chip in
+// one round, a launch lasts as long as one block: the most steps that still
+// fit, in the smallest region (fewer nodes of margin per wave).  us per step,
+// FP64 BGK / FP32 CM:
+//   128^2  24 x 24 regions, 8 steps 1.17 / 1.05; 32 x 32, 8 1.34 / 1.21
+//   192^2  24 x 24, 6 1.42 / 1.24;  32 x 32, 8 1.50 / 1.32
+//   256^2  32 x 32, 8 1.67 / 1.41;  6 steps 1.80 / 1.56
+//   320^2  32 x 32, 6 1.95 / 1.63;  8 steps (two rounds) 2.76 / 2.16
+//   384^2  32 x 32, 4 2.41 / 2.09;  6 steps 2.98 / 2.47, 8 3.67 / 2.95
+// with walls (cavity FP64 CM): 129^2 8 steps 3.7, 6 3.8, 4 4.5; 257^2 4.7, 5.6, 7.8.
+// Larger planes are bound by traffic and by the work on margins: 4-byte and
+// 2-byte populations take 64 x 32 regions and 6 steps (1024^2 FP32 7.9 us per
+// step, 8.0 at 4 steps, 9.3 with 32 x 32 regions, 11.1 one launch per step;
+// 4096^2 93, 96, 125 and 189), 8-byte ones 32 x 32 and 4 (1024^2 12.0 us, 12.2
+// at 6, 13.5 with 64 x 32 regions, 23.6 one launch per step; 4096^2 169 and 426).
+inline PlanePlan plane_rule(const PlaneBox& b) {
+  PlanePlan p;
+  p.nodes = b.nodes;
+  const bool walls = b.nodes == kPlaneWalls;
+  const int steps_shapes[5][2] = {{8, kPlaneSmall},  {6, kPlaneSmall}, {8, kPlaneSquare},
+                                  {6, kPlaneSquare}, {4, kPlaneSquare}};
+  for (const auto& c : steps_shapes) {
+    if (walls && c[1] == kPlaneSmall) continue;
+    const PlaneGrid g = plane_grid(b.sx, b.sy, c[0], c[1], b.nodes);
+    if (int64_t(g.ntx) * g.nty > b.cus) continue;
+    p.steps = c[0];
+    p.shape = c[1];
+    return p;
+  }
+  p.shape = kPlaneSquare;
+  if (walls || b.elem_bytes == 8) {
+    p.steps = 4;
+  } else {
+    p.shape = kPlaneWide;
+    p.steps = 6;
+    // 2-byte populations beyond the caches' reach of one XCD gain little (D2Q9
+    // CM 2048^2, us per step: FP16 27.2 against 27.3, BF16 25.7 / 28.1, I16
+    // 24.7 / 28.5), and E2M13 (32.0 / 30.6, its codec runs on the margins too)
+    // and boxes with geometry (FP16 28.2 / 27.6, E2M13 34.0 / 29.4) lose
+    if (b.elem_bytes == 2 && b.bytes > (32u << 20) && (b.e2m13 || b.nodes == kPlaneGeom))
+      p.steps = 0;
+  }
+  return p;
+}
+
+// ---- two D3Q27 steps per pass through LDS ----
+// Core of a block along x and y.
+constexpr RegionSize march_core(int elem_bytes) {
+  return elem_bytes == 8 ? RegionSize{32, 12} : RegionSize{64, 13};
+}
+
+struct MarchBox {
+  int sx, sy, sz;  // padded extents
+  int elem_bytes;
+  int cus;
+};
+
+struct MarchPlan {
+  bool on = false;
+  int ntx = 0, nty = 0, nzc = 0;  // blocks along x, y and z
+};
+
+// The blocks along z are chosen for the least rounds of blocks times planes of
+// one (two planes and about half a plane's time of start are extra).  on: that
+// schedule keeps the chip's cells filled.  GLUPS against the pass of pair.hpp,
+// 4-byte storage: 0.81 (192^3) 35.5 / 29.6, 0.65 (160^3) 28.3 / 28.9; 8-byte: 0.75
+// (150x130x140) 16.1 / 13.0, 0.58 (74x172x118) 12.5 / 9.9.
+inline MarchPlan march_rule(const MarchBox& b) {
+  MarchPlan p;
+  const RegionSize core = march_core(b.elem_bytes);
+  p.ntx = (b.sx + core.x - 1) / core.x;
+  p.nty = (b.sy + core.y - 1) / core.y;
+  const int64_t cols = int64_t(p.ntx) * p.nty;
+  double best = 0;
+  for (int k = 1; k <= b.sz; ++k) {
+    const double cost = double((cols * k + b.cus - 1) / b.cus) * ((b.sz + k - 1) / k + 2.5);
+    if (k == 1 || cost < best) {
+      best = cost;
+      p.nzc = k;
+    }
+  }
+  const double nodes = double(b.sx) * b.sy * b.sz;
+  p.on = nodes / (best * b.cus * core.x * core.y) >= (b.elem_bytes == 8 ? 0.5 : 0.65);
+  return p;
+}
+
+}  // namespace m3lb

@@ -1,0 +1,91 @@
+// Host checks of step_plan.hpp.  Prints "ok".
+#include "../../m3lb_amd/csrc/step_plan.hpp"
+
+#include <cstdio>
+#include <cstdlib>
+#include <string>
+
+using namespace m3lb;
+
+#define REQUIRE(x)                                \
+  do {                                            \
+    if (!(x)) {                                   \
+      std::printf("line %d: %s\n", __LINE__, #x); \
+      std::exit(1);                               \
+    }                                             \
+  } while (0)
+
+namespace {
+PlaneBox plane(int sx, int sy, int nodes, int elem_bytes, bool e2m13 = false) {
+  PlaneBox b{};
+  b.sx = sx;
+  b.sy = sy;
+  b.nodes = nodes;
+  b.elem_bytes = elem_bytes;
+  b.e2m13 = e2m13;
+  b.bytes = uint64_t(sx) * uint64_t(sy) * 9 * uint64_t(elem_bytes);
+  b.cus = 256;
+  return b;
+}
+
+// Squares: the steps and regions the rule's measurements name.
+void squares() {
+  const struct {
+    int n, elem_bytes, steps, shape;
+  } want[] = {{128, 8, 8, kPlaneSmall},  {128, 4, 8, kPlaneSmall},  {192, 8, 6, kPlaneSmall},
+              {256, 4, 8, kPlaneSquare}, {320, 8, 6, kPlaneSquare}, {384, 4, 4, kPlaneSquare},
+              {1024, 8, 4, kPlaneSquare}, {1024, 4, 6, kPlaneWide}, {1024, 2, 6, kPlaneWide},
+              {4096, 4, 6, kPlaneWide}};
+  for (const auto& w : want) {
+    const PlanePlan p = plane_rule(plane(w.n, w.n, kPlaneFluid, w.elem_bytes));
+    REQUIRE(p.steps == w.steps && p.shape == w.shape);
+  }
+  REQUIRE(plane_rule(plane(2048, 2048, kPlaneFluid, 2, true)).steps == 0);
+  REQUIRE(plane_rule(plane(2050, 2050, kPlaneGeom, 2)).steps == 0);
+  REQUIRE(plane_rule(plane(131, 131, kPlaneWalls, 8)).steps == 8);
+}
+
+// Every plan's cores cover the box, and its region holds a core and its margin.
+void covers() {
+  for (int nodes : {kPlaneFluid, kPlaneGeom, kPlaneWalls})
+    for (int eb : {8, 4, 2})
+      for (int sx : {1, 2, 7, 24, 65, 300, 1000, 70000})
+        for (int sy : {1, 3, 16, 33, 250, 900}) {
+          const PlanePlan p = plane_rule(plane(sx, sy, nodes, eb));
+          REQUIRE(p.steps % 2 == 0);
+          for (int n = 2; n <= p.steps; n += 2) {
+            const PlaneGrid g = plane_grid(sx, sy, n, p.shape, nodes);
+            const RegionSize r = plane_region(p.shape, nodes);
+            const int h = plane_margin(n, nodes);
+            REQUIRE(g.ntx >= 1 && g.nty >= 1 && g.ntx <= sx && g.nty <= sy);
+            REQUIRE((sx + g.ntx - 1) / g.ntx + 2 * h <= r.x);
+            REQUIRE((sy + g.nty - 1) / g.nty + 2 * h <= r.y);
+          }
+        }
+}
+
+void march() {
+  const struct {
+    int sx, sy, sz, elem_bytes;
+    bool on;
+  } want[] = {{512, 512, 512, 4, true}, {192, 192, 192, 4, true},  {150, 97, 121, 4, false},
+              {150, 130, 140, 8, true}, {300, 280, 260, 4, true}};
+  for (const auto& w : want) {
+    const MarchPlan p = march_rule({w.sx, w.sy, w.sz, w.elem_bytes, 256});
+    const RegionSize core = march_core(w.elem_bytes);
+    REQUIRE(p.on == w.on);
+    REQUIRE(p.nzc >= 1 && p.nzc <= w.sz && p.ntx * core.x >= w.sx);
+    REQUIRE((w.sy + p.nty - 1) / p.nty <= core.y);
+  }
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "squares") squares();
+  else if (what == "covers") covers();
+  else if (what == "march") march();
+  else return 2;
+  std::printf("ok\n");
+  return 0;
+}
