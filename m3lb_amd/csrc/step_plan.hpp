@@ -46,6 +46,33 @@ struct PlaneBox {
   int cus;
 };
 
+// Cells that a pass computes per node of the box and step: the margins, and what of
+// the regions' cores the box leaves empty.
+inline double plane_work(const PlaneBox& b, int steps, int shape) {
+  const PlaneGrid g = plane_grid(b.sx, b.sy, steps, shape, b.nodes);
+  const RegionSize r = plane_region(shape, b.nodes);
+  return double(g.ntx) * g.nty * r.x * r.y / (double(b.sx) * b.sy);
+}
+
+// Planes of more than four rounds of blocks (fewer: a one-launch step is bound by its
+// launch; 20000 x 4 FP64, 3.3 rounds, 1.46 times its speed), a few rows or columns
+// wide: a region then holds little of the box.  The one-launch step has lanes idle too in rows shorter
+// than a wave, so the work counts in proportion there.  Speed against one launch
+// per step, CM, work in brackets, 200,000 and 262,144 nodes long: 8-byte rows (4 steps)
+// 2 high (21) 0.46, 4 (11) 0.75-0.93, 8 (5.3) 0.99-1.24, 10 (4.3) 1.14-1.35, 18 (2.4) 1.3-
+// 1.8, columns of any width (1.7 or less) 1.5-2.6; 4-byte (6 steps) rows 2 high
+// 0.89, 4 (9.8) 0.81-0.96, 6 (6.6) 1.17, 8 (4.9) 1.33-1.5, columns up to 22 wide 0.8-0.97,
+// 26 1.04, 30 1.18, 44 2.2; FP16 rows 1 high 0.49, 2 (20) 0.6-0.93, 8 (4.9) 0.96-1.28, 24
+// (3.3) 0.89, 14 (2.8) 1.11-1.35, columns 60 wide (3.2) 0.71, 44 (1.6) 1.23; E2M13 rows 2
+// high 0.71, 8 0.95, 14 1.04.
+inline bool plane_fits(const PlaneBox& b, int steps, int shape) {
+  const PlaneGrid g = plane_grid(b.sx, b.sy, steps, shape, b.nodes);
+  if (int64_t(g.ntx) * g.nty <= 4 * b.cus) return true;
+  const double most = b.elem_bytes == 8 ? 5.0 : b.elem_bytes == 4 ? 6.6 : 2.9;
+  if (b.elem_bytes == 4 && b.sx < 26) return false;
+  return plane_work(b, steps, shape) * std::min(1.0, b.sx / 64.0) <= most;
+}
+
 struct PlanePlan {
   int steps = 0;  // most steps per launch, even; 0: one launch per step
   int shape = 0, nodes = 0;
@@ -93,6 +120,7 @@ inline PlanePlan plane_rule(const PlaneBox& b) {
     if (b.elem_bytes == 2 && b.bytes > (32u << 20) && (b.e2m13 || b.nodes == kPlaneGeom))
       p.steps = 0;
   }
+  if (p.steps && !walls && !plane_fits(b, p.steps, p.shape)) p.steps = 0;
   return p;
 }
 

@@ -64,6 +64,27 @@ void covers() {
         }
 }
 
+// Planes a few nodes thin and longer than one round of blocks: where a region holds
+// too little of the box, one launch per step.
+void thin() {
+  const struct {
+    int sx, sy, elem_bytes;
+    bool on;
+  } want[] = {{262144, 1, 8, false}, {262144, 4, 8, false}, {262144, 16, 8, true},
+              {4, 262144, 8, true},  {262144, 1, 4, false}, {262144, 4, 4, false},
+              {262144, 8, 4, true},  {4, 262144, 4, false}, {16, 262144, 4, false},
+              {48, 262144, 4, true}, {262144, 1, 2, false}, {262144, 4, 2, false},
+              {262144, 16, 2, true}, {60, 200000, 2, false}, {44, 200000, 2, true},
+              {800000000, 1, 4, false},
+              // few rounds: bound by launches
+              {20000, 4, 8, true},   {2000, 8, 4, true},    {3, 5000, 2, true}};
+  for (const auto& w : want) {
+    const PlanePlan p = plane_rule(plane(w.sx, w.sy, kPlaneFluid, w.elem_bytes));
+    if ((p.steps > 0) != w.on) std::printf("%d x %d, %d bytes\n", w.sx, w.sy, w.elem_bytes);
+    REQUIRE((p.steps > 0) == w.on);
+  }
+}
+
 void march() {
   const struct {
     int sx, sy, sz, elem_bytes;
@@ -84,6 +105,7 @@ int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "squares") squares();
   else if (what == "covers") covers();
+  else if (what == "thin") thin();
   else if (what == "march") march();
   else return 2;
   std::printf("ok\n");
