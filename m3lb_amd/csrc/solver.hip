@@ -880,6 +880,8 @@ m3lb::PlanePlan plane_plan(const m3lb_solver* s) {
   p.e2m13 = s->cfg.dtype == M3LB_E2M13;
   p.bytes = s->stride * uint64_t(s->Q) * uint64_t(s->ks->elem_bytes);
   p.cus = s->cus;
+  p.nwall = b.nwall;
+  p.corners = b.has_corners;
   return m3lb::plane_rule(p);
 }
 

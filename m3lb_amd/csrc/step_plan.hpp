@@ -5,6 +5,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 namespace m3lb {
@@ -44,6 +45,8 @@ struct PlaneBox {
   bool e2m13;
   uint64_t bytes;  // of the population array
   int cus;
+  int nwall;       // regularised wall nodes, and whether corners are among them
+  bool corners;
 };
 
 // Cells that a pass computes per node of the box and step: the margins, and what of
@@ -71,6 +74,38 @@ inline bool plane_fits(const PlaneBox& b, int steps, int shape) {
   const double most = b.elem_bytes == 8 ? 5.0 : b.elem_bytes == 4 ? 6.6 : 2.9;
   if (b.elem_bytes == 4 && b.sx < 26) return false;
   return plane_work(b, steps, shape) * std::min(1.0, b.sx / 64.0) <= most;
+}
+
+// us per step of a walled plane, one launch per step (two launches, with corners four) and
+// in passes of more than one round of blocks, and so the sizes up to which the passes
+// pay.  Within a round they always do.  Speed of the pass of 4 steps
+// against one launch per step, CM; channels (two straight walls): 500^2 FP64 1.15, FP32
+// 1.05, FP16 1.07, E2M13 0.87; 800^2 1.12, 0.81, 0.84, 0.70; 1600^2 0.85, 0.66, 0.44, 0.41;
+// 20000 x 40 0.80, 0.59, 0.47, 0.48; cavities: 500^2 1.99, 2.13, 2.03, 1.78; 800^2 1.63, 1.40,
+// 1.30, 1.13; 1100^2 1.26, 1.11, 0.93, 0.82; 2050^2 1.07, 0.69, 0.53, 0.46; 4100^2 FP64
+// 1.21.  The model names the faster way for 680 of 714 measured cases (five
+// storage types, 16 to 8000 nodes wide, 2 and 4 steps) and loses at most 8% to it
+// for the 8 others that it takes.
+inline double walled_one(const PlaneBox& b) {
+  const bool beyond = b.bytes > (256u << 20);  // the last-level cache
+  const double ps = b.elem_bytes == 8   ? (beyond ? 30.0 : 21.3)
+                    : b.elem_bytes == 4 ? (beyond ? 15.5 : 10.8)
+                    : b.e2m13           ? (beyond ? 8.7 : 7.6)
+                                        : (beyond ? 8.3 : 7.2);
+  const double start = b.elem_bytes == 8 ? 7.3 : b.elem_bytes == 4 ? 6.3 : 8.0;
+  return start + (b.corners ? 10.0 : 0.0) + double(b.sx) * b.sy * ps * 1e-6;
+}
+inline double walled_pass(const PlaneBox& b, int steps) {
+  const PlaneGrid g = plane_grid(b.sx, b.sy, steps, kPlaneSquare, kPlaneWalls);
+  const double blocks = double(g.ntx) * g.nty;
+  const bool two = steps == 2;
+  const double round = b.elem_bytes == 8   ? (two ? 6.8 : 8.8)
+                       : b.elem_bytes == 4 ? (two ? 4.9 : 6.7)
+                       : b.e2m13           ? (two ? 6.3 : 8.9)
+                                           : (two ? 5.6 : 7.7);
+  // a block with walls takes longer: its share, at 20 wall nodes a block
+  const double walled = std::min(1.0, b.nwall / (20.0 * blocks));
+  return (6.0 + std::ceil(blocks / b.cus) * (round + (two ? 2.5 : 3.4) * walled)) / steps;
 }
 
 struct PlanePlan {
@@ -120,7 +155,9 @@ inline PlanePlan plane_rule(const PlaneBox& b) {
     if (b.elem_bytes == 2 && b.bytes > (32u << 20) && (b.e2m13 || b.nodes == kPlaneGeom))
       p.steps = 0;
   }
-  if (p.steps && !walls && !plane_fits(b, p.steps, p.shape)) p.steps = 0;
+  if (walls ? walled_pass(b, p.steps) >= walled_one(b)
+            : p.steps && !plane_fits(b, p.steps, p.shape))
+    p.steps = 0;
   return p;
 }
 

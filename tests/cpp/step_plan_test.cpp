@@ -85,6 +85,36 @@ void thin() {
   }
 }
 
+// Walled planes beyond one round of blocks, the measured faster way.
+void walls() {
+  const struct {
+    int nx, ny;
+    bool cavity;
+    int elem_bytes;
+    bool e2m13, on;
+  } want[] = {{500, 500, false, 8, false, true},    {800, 800, false, 8, false, true},
+              {1600, 1600, false, 8, false, false}, {20000, 40, false, 8, false, false},
+              {500, 500, true, 8, false, true},     {1100, 1100, true, 8, false, true},
+              {4100, 4100, true, 8, false, true},   {500, 500, false, 4, false, true},
+              {800, 800, false, 4, false, false},   {1600, 1600, false, 4, false, false},
+              {800, 800, true, 4, false, true},     {2050, 2050, true, 4, false, false},
+              {800, 800, false, 2, false, false},   {800, 800, true, 2, false, true},
+              {1100, 1100, true, 2, false, false},  {1600, 1600, true, 2, false, false},
+              {500, 500, false, 2, true, false},    {600, 600, true, 2, true, true},
+              {1100, 1100, true, 2, true, false},
+              // within one round
+              {33, 33, true, 2, true, true},        {129, 129, true, 4, false, true},
+              {2000, 14, false, 2, true, true}};
+  for (const auto& w : want) {
+    PlaneBox b = plane(w.nx + (w.cavity ? 2 : 0), w.ny + 2, kPlaneWalls, w.elem_bytes, w.e2m13);
+    b.nwall = 2 * w.nx + (w.cavity ? 2 * w.ny - 4 : 0);
+    b.corners = w.cavity;
+    const PlanePlan p = plane_rule(b);
+    if ((p.steps > 0) != w.on) std::printf("%d x %d, %d bytes\n", w.nx, w.ny, w.elem_bytes);
+    REQUIRE((p.steps > 0) == w.on);
+  }
+}
+
 void march() {
   const struct {
     int sx, sy, sz, elem_bytes;
@@ -106,6 +136,7 @@ int main(int argc, char** argv) {
   if (what == "squares") squares();
   else if (what == "covers") covers();
   else if (what == "thin") thin();
+  else if (what == "walls") walls();
   else if (what == "march") march();
   else return 2;
   std::printf("ok\n");
