@@ -863,11 +863,11 @@ int launch_pair(m3lb_solver* s, const m3lb::StepArgs& a, int parity) {
 
 // Several steps of a plane box per launch (plane.hpp).  Applies to a box whose
 // moving nodes read no other node's set (no outlets, no specular cells, corner
-// stencils on walls) and unless fusion is off.
-m3lb::PlanePlan plane_plan(const m3lb_solver* s) {
+// stencils on walls) and unless fusion is off.  left: steps that passes may take.
+m3lb::PlanePlan plane_plan(const m3lb_solver* s, int left) {
   const Boundaries& b = s->b;
   const m3lb::Dom& d = s->d;
-  if (!s->ks->plane || s->fusion == M3LB_FUSION_OFF || s->alt_failed || s->Q != 9) return {};
+  if (left < 2 || !s->ks->plane || s->fusion == M3LB_FUSION_OFF || s->alt_failed || s->Q != 9) return {};
   if (b.nspec || b.nsnap || (b.nwall && !b.local)) return {};
   // an unwrapped axis without a halo (one node, not periodic) has no margin
   if (!(d.px || d.hx) || !(d.py || d.hy)) return {};
@@ -882,7 +882,8 @@ m3lb::PlanePlan plane_plan(const m3lb_solver* s) {
   p.cus = s->cus;
   p.nwall = b.nwall;
   p.corners = b.has_corners;
-  return m3lb::plane_rule(p);
+  p.force = s->cfg.forcing != M3LB_FORCE_NONE;
+  return m3lb::plane_rule(p, left);
 }
 
 // The second population array: allocated at the first pass, and given the
@@ -908,9 +909,9 @@ int ensure_alt(m3lb_solver* s, bool statics) {
   return M3LB_OK;
 }
 
-// `steps` (even) steps from an even one.
+// p.steps steps from an even one.
 int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& wa,
-                 const m3lb::PlanePlan& p, int steps) {
+                 const m3lb::PlanePlan& p) {
   m3lb::PlaneArgs pa;
   std::memset(&pa, 0, sizeof pa);
   pa.a = a;
@@ -918,9 +919,9 @@ int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& 
   for (int j = 0; j < 4; ++j) pa.a.macro[j] = nullptr;
   pa.w = wa;
   pa.out = s->f_alt;
-  pa.steps = steps;
-  pa.margin = m3lb::plane_margin(steps, p.nodes);
-  const m3lb::PlaneGrid g = m3lb::plane_grid(s->d.sx, s->d.sy, steps, p.shape, p.nodes);
+  pa.steps = p.steps;
+  pa.margin = m3lb::plane_margin(p.steps, p.nodes);
+  const m3lb::PlaneGrid g = m3lb::plane_grid(s->d.sx, s->d.sy, p.steps, p.shape, p.nodes);
   pa.ntx = g.ntx;
   pa.nty = g.nty;
   pa.core_x = s->d.sx / pa.ntx;
@@ -1063,8 +1064,8 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
     if (rc) return rc;
     if (s->alt_failed) march.on = false;
   }
-  m3lb::PlanePlan plane = plane_plan(s);
-  if (plane.steps && passable - int(s->t % 2) >= 2) {
+  m3lb::PlanePlan plane = plane_plan(s, passable - int(s->t % 2));
+  if (plane.steps) {
     const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid);
     if (rc) return rc;
     if (s->alt_failed) plane.steps = 0;
@@ -1074,9 +1075,10 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
     // the plane passes: even numbers of steps from an even one (never the
     // step that stores the macroscopic fields)
     const int left = nsteps - k - (store_macroscopic ? 1 : 0);
+    if (plane.steps > left) plane = plane_plan(s, left);  // the last, shorter pass
     if (plane.steps && left >= 2 && s->t % 2 == 0) {
-      const int n = std::min(plane.steps, left & ~1);
-      const int rc = launch_plane(s, a, wa, plane, n);
+      const int n = plane.steps;
+      const int rc = launch_plane(s, a, wa, plane);
       if (rc) return rc;
       a.f = wa.f = sa.f = s->f;
       na.f = s->f;

@@ -47,6 +47,7 @@ struct PlaneBox {
   int cus;
   int nwall;       // regularised wall nodes, and whether corners are among them
   bool corners;
+  bool force;
 };
 
 // Cells that a pass computes per node of the box and step: the margins, and what of
@@ -67,12 +68,17 @@ inline double plane_work(const PlaneBox& b, int steps, int shape) {
 // 0.89, 4 (9.8) 0.81-0.96, 6 (6.6) 1.17, 8 (4.9) 1.33-1.5, columns up to 22 wide 0.8-0.97,
 // 26 1.04, 30 1.18, 44 2.2; FP16 rows 1 high 0.49, 2 (20) 0.6-0.93, 8 (4.9) 0.96-1.28, 24
 // (3.3) 0.89, 14 (2.8) 1.11-1.35, columns 60 wide (3.2) 0.71, 44 (1.6) 1.23; E2M13 rows 2
-// high 0.71, 8 0.95, 14 1.04.
+// high 0.71, 8 0.95, 14 1.04.  Two steps bring less: 8-byte rows 10 high (3.7) 0.89-0.96,
+// 14 (2.6) 1.01-1.08; 4-byte rows 4 high (8.5) 0.68-0.87, 8 (4.3) 1.27, columns 36 wide 0.87-
+// 1.02, 44 1.5; FP16 rows 10 high (2.9) 0.93, 14 (2.1) 1.05.
 inline bool plane_fits(const PlaneBox& b, int steps, int shape) {
+  const bool two = steps == 2;
   const PlaneGrid g = plane_grid(b.sx, b.sy, steps, shape, b.nodes);
-  if (int64_t(g.ntx) * g.nty <= 4 * b.cus) return true;
-  const double most = b.elem_bytes == 8 ? 5.0 : b.elem_bytes == 4 ? 6.6 : 2.9;
-  if (b.elem_bytes == 4 && b.sx < 26) return false;
+  if (int64_t(g.ntx) * g.nty <= (two ? 2 : 4) * b.cus) return true;
+  const double most = b.elem_bytes == 8   ? (two ? 3.0 : 5.0)
+                      : b.elem_bytes == 4 ? (two ? 4.3 : 6.6)
+                                          : (two ? 2.2 : 2.9);
+  if (b.elem_bytes == 4 && b.sx < (two ? 40 : 26)) return false;
   return plane_work(b, steps, shape) * std::min(1.0, b.sx / 64.0) <= most;
 }
 
@@ -83,23 +89,25 @@ inline bool plane_fits(const PlaneBox& b, int steps, int shape) {
 // 1.05, FP16 1.07, E2M13 0.87; 800^2 1.12, 0.81, 0.84, 0.70; 1600^2 0.85, 0.66, 0.44, 0.41;
 // 20000 x 40 0.80, 0.59, 0.47, 0.48; cavities: 500^2 1.99, 2.13, 2.03, 1.78; 800^2 1.63, 1.40,
 // 1.30, 1.13; 1100^2 1.26, 1.11, 0.93, 0.82; 2050^2 1.07, 0.69, 0.53, 0.46; 4100^2 FP64
-// 1.21.  The model names the faster way for 680 of 714 measured cases (five
-// storage types, 16 to 8000 nodes wide, 2 and 4 steps) and loses at most 8% to it
-// for the 8 others that it takes.
+// 1.21.  A Guo force costs the FP64 pass most (800^2 channel, BGK: 23.4 us against 19.2).
+// The model names the faster way for 688 of 714 measured cases (five storage types, 16
+// to 8000 nodes wide, 2 and 4 steps); the four others that it gives to the passes are
+// at most 4% slower there.
 inline double walled_one(const PlaneBox& b) {
   const bool beyond = b.bytes > (256u << 20);  // the last-level cache
-  const double ps = b.elem_bytes == 8   ? (beyond ? 30.0 : 21.3)
+  const double ps = b.elem_bytes == 8   ? (!beyond ? 21.3 : b.bytes > (512u << 20) ? 30.0 : 26.0)
                     : b.elem_bytes == 4 ? (beyond ? 15.5 : 10.8)
                     : b.e2m13           ? (beyond ? 8.7 : 7.6)
                                         : (beyond ? 8.3 : 7.2);
   const double start = b.elem_bytes == 8 ? 7.3 : b.elem_bytes == 4 ? 6.3 : 8.0;
-  return start + (b.corners ? 10.0 : 0.0) + double(b.sx) * b.sy * ps * 1e-6;
+  return start + (b.corners ? 11.5 : 0.0) + double(b.sx) * b.sy * ps * 1e-6;
 }
 inline double walled_pass(const PlaneBox& b, int steps) {
   const PlaneGrid g = plane_grid(b.sx, b.sy, steps, kPlaneSquare, kPlaneWalls);
   const double blocks = double(g.ntx) * g.nty;
   const bool two = steps == 2;
-  const double round = b.elem_bytes == 8   ? (two ? 6.8 : 8.8)
+  const bool beyond = b.bytes > (256u << 20);
+  const double round = b.elem_bytes == 8   ? (two ? (beyond ? 7.2 : 6.8) : b.force ? 10.4 : 8.8)
                        : b.elem_bytes == 4 ? (two ? 4.9 : 6.7)
                        : b.e2m13           ? (two ? 6.3 : 8.9)
                                            : (two ? 5.6 : 7.7);
@@ -109,7 +117,7 @@ inline double walled_pass(const PlaneBox& b, int steps) {
 }
 
 struct PlanePlan {
-  int steps = 0;  // most steps per launch, even; 0: one launch per step
+  int steps = 0;  // of the next launch, even; 0: one launch per step
   int shape = 0, nodes = 0;
 };
 
@@ -128,7 +136,14 @@ struct PlanePlan {
 // step, 8.0 at 4 steps, 9.3 with 32 x 32 regions, 11.1 one launch per step;
 // 4096^2 93, 96, 125 and 189), 8-byte ones 32 x 32 and 4 (1024^2 12.0 us, 12.2
 // at 6, 13.5 with 64 x 32 regions, 23.6 one launch per step; 4096^2 169 and 426).
-inline PlanePlan plane_rule(const PlaneBox& b) {
+// left: the steps that are left for passes.  A pass of two steps has cores of
+// 60 x 28 nodes in 64 x 32 regions: up to two rounds of such blocks the 32 x 32
+// regions, with twice the blocks, keep more of the chip at work (speed against
+// one launch per step, 64 x 32 / 32 x 32: 400x390 FP32 0.92 / 1.28, with geometry 0.66 /
+// 1.16, 520x510 0.79 / 1.11, 700x690 0.98 / 1.18; 1024x1014 1.12 / 1.11, FP16 1.30 / 1.06),
+// and E2M13 loses in either (520x510 0.97 / 0.99, with geometry 0.68 / 0.90, 700x690
+// 0.86 / 0.94, 1024x1014 0.97 / 0.81).
+inline PlanePlan plane_rule(const PlaneBox& b, int left) {
   PlanePlan p;
   p.nodes = b.nodes;
   const bool walls = b.nodes == kPlaneWalls;
@@ -136,18 +151,24 @@ inline PlanePlan plane_rule(const PlaneBox& b) {
                                   {6, kPlaneSquare}, {4, kPlaneSquare}};
   for (const auto& c : steps_shapes) {
     if (walls && c[1] == kPlaneSmall) continue;
-    const PlaneGrid g = plane_grid(b.sx, b.sy, c[0], c[1], b.nodes);
+    const int steps = std::min(c[0], left & ~1);
+    const PlaneGrid g = plane_grid(b.sx, b.sy, steps, c[1], b.nodes);
     if (int64_t(g.ntx) * g.nty > b.cus) continue;
-    p.steps = c[0];
+    p.steps = steps;
     p.shape = c[1];
     return p;
   }
   p.shape = kPlaneSquare;
   if (walls || b.elem_bytes == 8) {
-    p.steps = 4;
+    p.steps = std::min(4, left & ~1);
   } else {
     p.shape = kPlaneWide;
-    p.steps = 6;
+    p.steps = std::min(6, left & ~1);
+    if (p.steps == 2) {
+      const PlaneGrid g = plane_grid(b.sx, b.sy, 2, kPlaneWide, b.nodes);
+      if (int64_t(g.ntx) * g.nty <= 2 * b.cus) p.shape = kPlaneSquare;
+      if (b.e2m13) p.steps = 0;
+    }
     // 2-byte populations beyond the caches' reach of one XCD gain little (D2Q9
     // CM 2048^2, us per step: FP16 27.2 against 27.3, BF16 25.7 / 28.1, I16
     // 24.7 / 28.5), and E2M13 (32.0 / 30.6, its codec runs on the margins too)
@@ -155,7 +176,7 @@ inline PlanePlan plane_rule(const PlaneBox& b) {
     if (b.elem_bytes == 2 && b.bytes > (32u << 20) && (b.e2m13 || b.nodes == kPlaneGeom))
       p.steps = 0;
   }
-  if (walls ? walled_pass(b, p.steps) >= walled_one(b)
+  if (walls ? walled_pass(b, p.steps) >= 0.97 * walled_one(b)
             : p.steps && !plane_fits(b, p.steps, p.shape))
     p.steps = 0;
   return p;

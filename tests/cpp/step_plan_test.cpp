@@ -37,12 +37,12 @@ void squares() {
               {1024, 8, 4, kPlaneSquare}, {1024, 4, 6, kPlaneWide}, {1024, 2, 6, kPlaneWide},
               {4096, 4, 6, kPlaneWide}};
   for (const auto& w : want) {
-    const PlanePlan p = plane_rule(plane(w.n, w.n, kPlaneFluid, w.elem_bytes));
+    const PlanePlan p = plane_rule(plane(w.n, w.n, kPlaneFluid, w.elem_bytes), 100);
     REQUIRE(p.steps == w.steps && p.shape == w.shape);
   }
-  REQUIRE(plane_rule(plane(2048, 2048, kPlaneFluid, 2, true)).steps == 0);
-  REQUIRE(plane_rule(plane(2050, 2050, kPlaneGeom, 2)).steps == 0);
-  REQUIRE(plane_rule(plane(131, 131, kPlaneWalls, 8)).steps == 8);
+  REQUIRE(plane_rule(plane(2048, 2048, kPlaneFluid, 2, true), 100).steps == 0);
+  REQUIRE(plane_rule(plane(2050, 2050, kPlaneGeom, 2), 100).steps == 0);
+  REQUIRE(plane_rule(plane(131, 131, kPlaneWalls, 8), 100).steps == 8);
 }
 
 // Every plan's cores cover the box, and its region holds a core and its margin.
@@ -51,12 +51,15 @@ void covers() {
     for (int eb : {8, 4, 2})
       for (int sx : {1, 2, 7, 24, 65, 300, 1000, 70000})
         for (int sy : {1, 3, 16, 33, 250, 900}) {
-          const PlanePlan p = plane_rule(plane(sx, sy, nodes, eb));
-          REQUIRE(p.steps % 2 == 0);
-          for (int n = 2; n <= p.steps; n += 2) {
-            const PlaneGrid g = plane_grid(sx, sy, n, p.shape, nodes);
+          for (int left = 2; left <= 12; ++left) {
+            const PlanePlan p = plane_rule(plane(sx, sy, nodes, eb), left);
+            REQUIRE(p.steps % 2 == 0 && p.steps <= left);
+            if (!p.steps) continue;
+            const PlaneGrid g = plane_grid(sx, sy, p.steps, p.shape, nodes);
             const RegionSize r = plane_region(p.shape, nodes);
-            const int h = plane_margin(n, nodes);
+            const int h = plane_margin(p.steps, nodes);
+            REQUIRE(p.shape != kPlaneWide || eb <= 4);  // no such kernel for 8-byte storage
+            REQUIRE(nodes != kPlaneWalls || p.shape == kPlaneSquare);
             REQUIRE(g.ntx >= 1 && g.nty >= 1 && g.ntx <= sx && g.nty <= sy);
             REQUIRE((sx + g.ntx - 1) / g.ntx + 2 * h <= r.x);
             REQUIRE((sy + g.nty - 1) / g.nty + 2 * h <= r.y);
@@ -79,7 +82,7 @@ void thin() {
               // few rounds: bound by launches
               {20000, 4, 8, true},   {2000, 8, 4, true},    {3, 5000, 2, true}};
   for (const auto& w : want) {
-    const PlanePlan p = plane_rule(plane(w.sx, w.sy, kPlaneFluid, w.elem_bytes));
+    const PlanePlan p = plane_rule(plane(w.sx, w.sy, kPlaneFluid, w.elem_bytes), 100);
     if ((p.steps > 0) != w.on) std::printf("%d x %d, %d bytes\n", w.sx, w.sy, w.elem_bytes);
     REQUIRE((p.steps > 0) == w.on);
   }
@@ -109,9 +112,30 @@ void walls() {
     PlaneBox b = plane(w.nx + (w.cavity ? 2 : 0), w.ny + 2, kPlaneWalls, w.elem_bytes, w.e2m13);
     b.nwall = 2 * w.nx + (w.cavity ? 2 * w.ny - 4 : 0);
     b.corners = w.cavity;
-    const PlanePlan p = plane_rule(b);
+    const PlanePlan p = plane_rule(b, 100);
     if ((p.steps > 0) != w.on) std::printf("%d x %d, %d bytes\n", w.nx, w.ny, w.elem_bytes);
     REQUIRE((p.steps > 0) == w.on);
+  }
+}
+
+// Passes of two steps: the region by the blocks it gives, and where one launch per
+// step is faster.
+void two_steps() {
+  const struct {
+    int n, nodes, elem_bytes;
+    bool e2m13;
+    int steps, shape;
+  } want[] = {{400, kPlaneFluid, 4, false, 2, kPlaneSquare}, {400, kPlaneGeom, 2, false, 2, kPlaneSquare},
+              {700, kPlaneGeom, 4, false, 2, kPlaneSquare},  {1024, kPlaneFluid, 4, false, 2, kPlaneWide},
+              {1024, kPlaneGeom, 2, false, 2, kPlaneWide},   {400, kPlaneGeom, 2, true, 2, kPlaneSquare},
+              {520, kPlaneGeom, 2, true, 0, 0},              {1024, kPlaneFluid, 2, true, 0, 0},
+              {1024, kPlaneFluid, 8, false, 2, kPlaneSquare}, {100, kPlaneFluid, 8, false, 2, kPlaneSmall}};
+  for (const auto& w : want) {
+    for (int left : {2, 3}) {
+      const PlanePlan p = plane_rule(plane(w.n, w.n, w.nodes, w.elem_bytes, w.e2m13), left);
+      if (p.steps != w.steps) std::printf("%d^2, %d bytes, %d steps\n", w.n, w.elem_bytes, p.steps);
+      REQUIRE(p.steps == w.steps && (!w.steps || p.shape == w.shape));
+    }
   }
 }
 
@@ -137,6 +161,7 @@ int main(int argc, char** argv) {
   else if (what == "covers") covers();
   else if (what == "thin") thin();
   else if (what == "walls") walls();
+  else if (what == "two_steps") two_steps();
   else if (what == "march") march();
   else return 2;
   std::printf("ok\n");
