@@ -211,7 +211,9 @@ inline MarchPlan march_rule(const MarchBox& b) {
   p.nty = (b.sy + core.y - 1) / core.y;
   const int64_t cols = int64_t(p.ntx) * p.nty;
   double best = 0;
-  for (int k = 1; k <= b.sz; ++k) {
+  // 4096 runs are 16 rounds of one column's blocks; a box of more planes than that
+  // gains nothing from more, and is not to be searched plane by plane each call
+  for (int k = 1; k <= std::min(b.sz, 4096); ++k) {
     const double cost = double((cols * k + b.cus - 1) / b.cus) * ((b.sz + k - 1) / k + 2.5);
     if (k == 1 || cost < best) {
       best = cost;

@@ -1,6 +1,7 @@
 // Host checks of step_plan.hpp.  Prints "ok".
 #include "../../m3lb_amd/csrc/step_plan.hpp"
 
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <string>
@@ -153,6 +154,16 @@ void march() {
     REQUIRE((w.sy + p.nty - 1) / p.nty <= core.y);
   }
 }
+// The rule runs at each step call: its cost does not grow with the box.
+void long_boxes() {
+  const auto t0 = std::chrono::steady_clock::now();
+  int on = 0;
+  for (int k = 0; k < 200; ++k) on += march_rule({4, 4, 10000000 + k, 4, 256}).on;
+  const double s =
+      std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  if (s > 1.0) std::printf("%.3f s for 200 calls\n", s);
+  REQUIRE(on == 0 && s <= 1.0);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -163,6 +174,7 @@ int main(int argc, char** argv) {
   else if (what == "walls") walls();
   else if (what == "two_steps") two_steps();
   else if (what == "march") march();
+  else if (what == "long_boxes") long_boxes();
   else return 2;
   std::printf("ok\n");
   return 0;

@@ -17,7 +17,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["squares", "covers", "thin", "walls", "two_steps", "march"])
+@pytest.mark.parametrize("case", ["squares", "covers", "thin", "walls", "two_steps", "march",
+                                  "long_boxes"])
 def test_step_plan(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
