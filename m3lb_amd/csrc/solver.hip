@@ -948,7 +948,8 @@ m3lb::MarchPlan march_plan(const m3lb_solver* s, const m3lb::StepArgs& a) {
     return {};
   // an unwrapped axis without a halo (one node, not periodic) has no margin
   if (!(d.px || d.hx) || !(d.py || d.hy) || !(d.pz || d.hz)) return {};
-  m3lb::MarchPlan p = m3lb::march_rule({d.sx, d.sy, d.sz, s->ks->elem_bytes, s->cus});
+  m3lb::MarchPlan p = m3lb::march_rule(
+      {d.sx, d.sy, d.sz, s->ks->elem_bytes, s->cus, s->geometry || d.hx || d.hy || d.hz});
   p.on = p.on || s->march_test;
   return p;
 }

@@ -182,7 +182,7 @@ inline PlanePlan plane_rule(const PlaneBox& b, int left) {
   return p;
 }
 
-// ---- two D3Q27 steps per pass through LDS ----
+// ---- two D3Q27 steps per pass through LDS (march.hpp) ----
 // Core of a block along x and y.
 constexpr RegionSize march_core(int elem_bytes) {
   return elem_bytes == 8 ? RegionSize{32, 12} : RegionSize{64, 13};
@@ -192,6 +192,7 @@ struct MarchBox {
   int sx, sy, sz;  // padded extents
   int elem_bytes;
   int cus;
+  bool geom;       // some node of the padded box is not Fluid
 };
 
 struct MarchPlan {
@@ -199,29 +200,53 @@ struct MarchPlan {
   int ntx = 0, nty = 0, nzc = 0;  // blocks along x, y and z
 };
 
-// The blocks along z are chosen for the least rounds of blocks times planes of
-// one (two planes and about half a plane's time of start are extra).  on: that
-// schedule keeps the chip's cells filled.  GLUPS against the pass of pair.hpp,
+// The runs along z with the least rounds of blocks times planes of one (two planes
+// and about half a plane's time of start are extra), none longer than `longest`.
+inline double march_runs(const MarchBox& b, int longest, MarchPlan& p) {
+  const int64_t cols = int64_t(p.ntx) * p.nty;
+  const int first = (b.sz + longest - 1) / longest;
+  // 4096 runs are 16 rounds of one column's blocks; a box of more planes than that
+  // gains nothing from more, and is not to be searched plane by plane each call
+  const int last = int(std::min<int64_t>(b.sz, int64_t(first) + 4095));
+  double best = 0;
+  for (int k = first; k <= last; ++k) {
+    const double cost = double((cols * k + b.cus - 1) / b.cus) * ((b.sz + k - 1) / k + 2.5);
+    if (k == first || cost < best) {
+      best = cost;
+      p.nzc = k;
+    }
+  }
+  return best;
+}
+
+// on: the schedule keeps the chip's cells filled.  GLUPS against the pass of pair.hpp,
 // 4-byte storage: 0.81 (192^3) 35.5 / 29.6, 0.65 (160^3) 28.3 / 28.9; 8-byte: 0.75
 // (150x130x140) 16.1 / 13.0, 0.58 (74x172x118) 12.5 / 9.9.
+//
+// Blocks of long runs drift apart in z, and with them the lines and margins that
+// neighbours share leave the caches before the neighbour comes: it shows where some
+// blocks are slower than others (geometry), beyond 120 planes: 11 of 11 FP64 boxes with a
+// halo at 0.79-1.02 of the speed of the pass of pair.hpp; with runs of up to 48
+// planes 288x320x256 0.86 -> 1.09, 300x280x260 0.80 -> 1.04, 445x213x159 0.96 -> 1.10,
+// 188x163x833 0.86 -> 1.03, 576x320x192 FP32 0.90 -> 1.08.  And where rows are no whole
+// half lines and the last core of a row is short, in FP32 rows of up to 256 nodes,
+// which the pass of pair.hpp takes in one tile: with runs of up to 16 planes 217x414x219 0.87 ->
+// 1.01, 147x535x285 0.85 -> 1.08, 156x349x440 0.88 -> 1.06, 100x400x400 0.99 -> 1.10 (runs of
+// up to 26 planes did not lose: 194x299x249 1.06, with 16 1.01).
 inline MarchPlan march_rule(const MarchBox& b) {
   MarchPlan p;
   const RegionSize core = march_core(b.elem_bytes);
   p.ntx = (b.sx + core.x - 1) / core.x;
   p.nty = (b.sy + core.y - 1) / core.y;
-  const int64_t cols = int64_t(p.ntx) * p.nty;
-  double best = 0;
-  // 4096 runs are 16 rounds of one column's blocks; a box of more planes than that
-  // gains nothing from more, and is not to be searched plane by plane each call
-  for (int k = 1; k <= std::min(b.sz, 4096); ++k) {
-    const double cost = double((cols * k + b.cus - 1) / b.cus) * ((b.sz + k - 1) / k + 2.5);
-    if (k == 1 || cost < best) {
-      best = cost;
-      p.nzc = k;
-    }
-  }
+  const double best = march_runs(b, b.sz, p);
   const double nodes = double(b.sx) * b.sy * b.sz;
   p.on = nodes / (best * b.cus * core.x * core.y) >= (b.elem_bytes == 8 ? 0.5 : 0.65);
+  const int run = (b.sz + p.nzc - 1) / p.nzc;
+  if (b.elem_bytes == 4 && b.sx <= 256 && b.sx % 16 != 0 && b.sx < 0.92 * core.x * p.ntx) {
+    if (run > 26) march_runs(b, 16, p);
+  } else if (b.geom && run > 120) {
+    march_runs(b, 48, p);
+  }
   return p;
 }
 

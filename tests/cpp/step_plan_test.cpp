@@ -147,18 +147,39 @@ void march() {
   } want[] = {{512, 512, 512, 4, true}, {192, 192, 192, 4, true},  {150, 97, 121, 4, false},
               {150, 130, 140, 8, true}, {300, 280, 260, 4, true}};
   for (const auto& w : want) {
-    const MarchPlan p = march_rule({w.sx, w.sy, w.sz, w.elem_bytes, 256});
+    const MarchPlan p = march_rule({w.sx, w.sy, w.sz, w.elem_bytes, 256, false});
     const RegionSize core = march_core(w.elem_bytes);
     REQUIRE(p.on == w.on);
     REQUIRE(p.nzc >= 1 && p.nzc <= w.sz && p.ntx * core.x >= w.sx);
     REQUIRE((w.sy + p.nty - 1) / p.nty <= core.y);
   }
 }
+// Longest runs of planes: short where blocks drift apart.
+void runs() {
+  const struct {
+    int sx, sy, sz, elem_bytes;
+    bool geom;
+    int longest;
+  } want[] = {{288, 322, 256, 8, true, 48},   {288, 320, 256, 8, false, 256},
+              {576, 322, 192, 4, true, 48},   {512, 512, 512, 4, false, 128},
+              {217, 414, 219, 4, false, 16},  {100, 400, 400, 4, false, 16},
+              {100, 402, 400, 4, true, 16},   {176, 419, 248, 4, false, 50},
+              {192, 192, 192, 4, false, 192}, {256, 258, 256, 4, true, 120}};
+  for (const auto& w : want) {
+    const MarchPlan p = march_rule({w.sx, w.sy, w.sz, w.elem_bytes, 256, w.geom});
+    const int run = (w.sz + p.nzc - 1) / p.nzc;
+    if (run > w.longest) std::printf("%d x %d x %d: runs of %d\n", w.sx, w.sy, w.sz, run);
+    REQUIRE(p.on && run <= w.longest);
+    if (w.longest >= 50 && run <= 16) std::printf("%d x %d x %d: runs of %d\n", w.sx, w.sy, w.sz, run);
+    if (w.longest >= 50) REQUIRE(run > 16);  // not shorter than it has to be
+  }
+}
+
 // The rule runs at each step call: its cost does not grow with the box.
 void long_boxes() {
   const auto t0 = std::chrono::steady_clock::now();
   int on = 0;
-  for (int k = 0; k < 200; ++k) on += march_rule({4, 4, 10000000 + k, 4, 256}).on;
+  for (int k = 0; k < 200; ++k) on += march_rule({4, 4, 10000000 + k, 4, 256, true}).on;
   const double s =
       std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   if (s > 1.0) std::printf("%.3f s for 200 calls\n", s);
@@ -174,6 +195,7 @@ int main(int argc, char** argv) {
   else if (what == "walls") walls();
   else if (what == "two_steps") two_steps();
   else if (what == "march") march();
+  else if (what == "runs") runs();
   else if (what == "long_boxes") long_boxes();
   else return 2;
   std::printf("ok\n");

@@ -17,7 +17,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["squares", "covers", "thin", "walls", "two_steps", "march",
+@pytest.mark.parametrize("case", ["squares", "covers", "thin", "walls", "two_steps", "march", "runs",
                                   "long_boxes"])
 def test_step_plan(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=120)
