@@ -135,7 +135,7 @@ struct m3lb_solver {
   // array and write the other; alt_synced: the slots that no moving node ever
   // writes hold the same values in both
   void* f_alt = nullptr;
-  bool alt_synced = false, alt_failed = false;
+  bool alt_synced = false;
   uint64_t stride = 0;  // elements per direction
   uint8_t* flags_d = nullptr;
   std::vector<uint8_t> flags_h;
@@ -867,7 +867,7 @@ int launch_pair(m3lb_solver* s, const m3lb::StepArgs& a, int parity) {
 m3lb::PlanePlan plane_plan(const m3lb_solver* s, int left) {
   const Boundaries& b = s->b;
   const m3lb::Dom& d = s->d;
-  if (left < 2 || !s->ks->plane || s->fusion == M3LB_FUSION_OFF || s->alt_failed || s->Q != 9) return {};
+  if (left < 2 || !s->ks->plane || s->fusion == M3LB_FUSION_OFF || s->Q != 9) return {};
   if (b.nspec || b.nsnap || (b.nwall && !b.local)) return {};
   // an unwrapped axis without a halo (one node, not periodic) has no margin
   if (!(d.px || d.hx) || !(d.py || d.hy)) return {};
@@ -887,9 +887,11 @@ m3lb::PlanePlan plane_plan(const m3lb_solver* s, int left) {
 }
 
 // The second population array: allocated at the first pass, and given the
-// slots no moving node writes whenever those may have changed.  Where there is
-// no room for it the box is left to one launch per step.
-int ensure_alt(m3lb_solver* s, bool statics) {
+// slots no moving node writes whenever those may have changed.  *have: false where
+// there is no room for it now; the steps of this call go another way, and the next
+// call asks again.
+int ensure_alt(m3lb_solver* s, bool statics, bool* have) {
+  *have = true;
   const size_t bytes = size_t(s->stride) * size_t(s->Q) * size_t(s->ks->elem_bytes);
   if (!s->f_alt) {
     // at most a quarter of what is free: other boxes keep room of their own
@@ -898,7 +900,7 @@ int ensure_alt(m3lb_solver* s, bool statics) {
         hipMalloc(&s->f_alt, bytes) != hipSuccess) {
       (void)hipGetLastError();
       s->f_alt = nullptr;
-      s->alt_failed = true;
+      *have = false;
       return M3LB_OK;
     }
     s->alt_synced = false;
@@ -941,7 +943,7 @@ int launch_plane(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::WallArgs& 
 // values of pair.hpp, that pass runs.
 m3lb::MarchPlan march_plan(const m3lb_solver* s, const m3lb::StepArgs& a) {
   const m3lb::Dom& d = s->d;
-  if (!s->ks->march || s->fusion != M3LB_FUSION_AUTO || s->alt_failed) return {};
+  if (!s->ks->march || s->fusion != M3LB_FUSION_AUTO) return {};
   if (s->b.nwall || s->b.nspec || s->b.nsnap) return {};
   if (!s->march_test &&
       (a.cached || s->pair_stripes || s->pair_lag || s->pair_bpc || s->pair_group))
@@ -1061,15 +1063,15 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   const int passable = nsteps - (store_macroscopic ? 1 : 0);
   if (march.on && pairs && s->t % 2 == 1 && passable % 2 == 0 && passable < 10) march.on = false;
   if (march.on && passable - int(s->t % 2) >= 2) {
-    const int rc = ensure_alt(s, s->geometry || s->d.hx || s->d.hy || s->d.hz);
+    const int rc = ensure_alt(s, s->geometry || s->d.hx || s->d.hy || s->d.hz, &march.on);
     if (rc) return rc;
-    if (s->alt_failed) march.on = false;
   }
   m3lb::PlanePlan plane = plane_plan(s, passable - int(s->t % 2));
   if (plane.steps) {
-    const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid);
+    bool have = false;
+    const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid, &have);
     if (rc) return rc;
-    if (s->alt_failed) plane.steps = 0;
+    if (!have) plane.steps = 0;
   }
   for (int k = 0; k < nsteps; ++k) {
     const bool last = k == nsteps - 1;

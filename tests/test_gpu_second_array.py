@@ -1,0 +1,81 @@
+"""The second population array of the passes on a device that is nearly full: most
+of the memory is held by plain allocations while these tests run."""
+import contextlib
+import ctypes
+
+import numpy as np
+import pytest
+
+from m3lb_amd import abi, solver
+from m3lb_amd.solver import FluidSolver
+
+pytestmark = pytest.mark.gpu
+
+PLANE = abi.make_config(abi.D2Q9, abi.OP_CM, abi.SHIFTED, abi.F64, (1300, 1200, 1), omega=1.6)
+BOX = abi.make_config(abi.D3Q27, abi.OP_CM, abi.SHIFTED, abi.F32, (192, 182, 190), omega=1.6)
+
+
+@pytest.fixture(autouse=True)
+def announce(request):
+    print(f"\n[gpu-case] {request.node.name}", flush=True)
+    yield
+
+
+def free_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert solver.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@contextlib.contextmanager
+def nearly_full(leave):
+    """All of the device's free memory but about `leave` bytes, held for a while."""
+    hip = solver.load()  # its dependency libamdhip64 resolves the entry points
+    held = []
+    try:
+        for _ in range(4):  # what is free after an allocation is not exactly the rest
+            n = free_bytes() - int(leave)
+            if n < (8 << 20):
+                break
+            p = ctypes.c_void_p()
+            assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(n)) == 0
+            held.append(p)
+        assert abs(free_bytes() - leave) < (16 << 20)
+        yield
+    finally:
+        for p in held:
+            assert hip.hipFree(p) == 0
+
+
+def init(s, cfg):
+    if cfg.lattice == abi.D3Q27:
+        s.initialize_taylor_green(0.04)
+    else:
+        s.initialize(1.0, 0.03, -0.02)
+    return s.device_bytes()
+
+
+def steps_of(cfg, counts):
+    with FluidSolver(cfg) as s:
+        s.set_step_fusion(abi.FUSION_OFF)
+        init(s, cfg)
+        for n in counts:
+            s.step(n)
+        return np.stack(s.compute_macroscopic())
+
+
+@pytest.mark.parametrize("cfg", [PLANE, BOX], ids=["plane", "box"])
+def test_no_room_now_and_room_later(cfg):
+    counts = (4, 6, 8)
+    want = steps_of(cfg, counts)
+    with FluidSolver(cfg) as s:
+        base = init(s, cfg)
+        with nearly_full(2 * base):  # more than the array, which may take a quarter
+            s.step(counts[0])
+            assert s.device_bytes() < 1.5 * base
+            if cfg.lattice == abi.D3Q27:
+                assert s.fused_passes() == 2  # in place
+        s.step(counts[1])
+        assert s.device_bytes() > 1.5 * base
+        s.step(counts[2])
+        assert np.array_equal(np.stack(s.compute_macroscopic()), want)
