@@ -2,8 +2,9 @@
 
 Fourteen instantiation units (one per lattice x collision operator, from
 csrc/inst.hip), the C-ABI unit of the single-box solver (csrc/solver.hip), the
-batched server (csrc/serve.hip) and the staged transfers (csrc/transfer.hip) compile in parallel into build objects under
-m3lb_amd/_build/, then link into m3lb_amd/libm3lb_hip.so.  Every HIP line
+batched server (csrc/serve.hip), the staged transfers (csrc/transfer.hip) and the
+device allocations (csrc/device_memory.hip) compile in parallel into build objects
+under m3lb_amd/_build/, then link into m3lb_amd/libm3lb_hip.so.  Every HIP line
 carries -Xclang -target-feature -Xclang -packed-fp32-ops: hipcc then emits no
 packed FP32 instructions.
 """
@@ -78,7 +79,7 @@ def build(force=True, jobs=None, verbose=False):
             cmds.append([HIPCC] + FLAGS + [f"-DM3LB_Q={q}", f"-DM3LB_OP={op}", "-c",
                                            os.path.join(CSRC, "inst.hip"), "-o", o])
     every = headers + [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip")]
-    for unit in ("solver", "serve", "transfer"):
+    for unit in ("solver", "serve", "transfer", "device_memory"):
         o = os.path.join(OBJ, f"{unit}.o")
         objs.append(o)
         # the C-ABI unit carries the build id, so it is rebuilt when any source changes

@@ -22,6 +22,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "device_memory.hpp"
 #include "launch.hpp"
 #include "serve_plan.hpp"
 #include "scales.hpp"
@@ -692,7 +693,7 @@ int m3lb_srv_create(const m3lb_server_config* cfg, m3lb_server** out) {
     return bail(err(M3LB_EDEVICE, "device attribute query failed"));
   s->grid = unsigned(s->cus * cfg->blocks_per_cu + 7) / 8 * 8;
   if (hipStreamCreate(&s->stream) != hipSuccess) return bail(err(M3LB_EDEVICE, "hipStreamCreate failed"));
-  if (hipMalloc(&s->arena_d, cfg->budget_bytes) != hipSuccess)
+  if (m3lb::device_alloc(s->device, &s->arena_d, cfg->budget_bytes) != hipSuccess)
     return bail(err(M3LB_ENOMEM, "arena: hipMalloc of " + std::to_string(cfg->budget_bytes) + " bytes failed"));
   s->arena.reset(cfg->budget_bytes);
   const size_t nb = size_t(cfg->max_boxes);
@@ -702,14 +703,14 @@ int m3lb_srv_create(const m3lb_server_config* cfg, m3lb_server** out) {
     if (hipHostMalloc(reinterpret_cast<void**>(&s->desc_h[k]), nb * sizeof(BoxDesc), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&s->hdr_h[k]), m3lb::pack_words(nb, kMaxChunk) * sizeof(unsigned), hipHostMallocDefault) != hipSuccess)
       return bail(err(M3LB_ENOMEM, "pinned descriptor buffers"));
-    if (hipMalloc(&s->desc_d[k], nb * sizeof(BoxDesc)) != hipSuccess ||
-        hipMalloc(&s->hdr_d[k], m3lb::pack_words(nb, kMaxChunk) * sizeof(unsigned)) != hipSuccess)
+    if (m3lb::device_alloc(s->device, &s->desc_d[k], nb * sizeof(BoxDesc)) != hipSuccess ||
+        m3lb::device_alloc(s->device, &s->hdr_d[k], m3lb::pack_words(nb, kMaxChunk) * sizeof(unsigned)) != hipSuccess)
       return bail(err(M3LB_ENOMEM, "device descriptor buffers"));
   }
   // completion sums (4 per block) and, for 16-bit storage, the largest
   // |g_q| per block at seeding (Q per block)
-  if (hipMalloc(&s->partial_d, kSumGrid * 27 * sizeof(double)) != hipSuccess ||
-      hipMalloc(&s->summary_d, nb * 4 * sizeof(double)) != hipSuccess ||
+  if (m3lb::device_alloc(s->device, &s->partial_d, kSumGrid * 27 * sizeof(double)) != hipSuccess ||
+      m3lb::device_alloc(s->device, &s->summary_d, nb * 4 * sizeof(double)) != hipSuccess ||
       hipHostMalloc(reinterpret_cast<void**>(&s->summary_h), nb * 4 * sizeof(double), hipHostMallocDefault) != hipSuccess)
     return bail(err(M3LB_ENOMEM, "summary buffers"));
   s->free_slots.reserve(nb);

@@ -12,6 +12,7 @@
 #include <string>
 #include <vector>
 
+#include "device_memory.hpp"
 #include "launch.hpp"
 #include "scales.hpp"
 #include "transfer.hpp"
@@ -136,6 +137,9 @@ struct m3lb_solver {
   // writes hold the same values in both
   void* f_alt = nullptr;
   bool alt_synced = false;
+  // held while a call uses f_alt: another handle's allocation may take it back
+  // between calls (device_memory.hpp)
+  mutable std::mutex alt_mu;
   uint64_t stride = 0;  // elements per direction
   uint8_t* flags_d = nullptr;
   std::vector<uint8_t> flags_h;
@@ -194,7 +198,7 @@ int ensure_partials(m3lb_solver* s, size_t n_doubles) {
   if (s->partial_n >= n_doubles) return M3LB_OK;
   if (s->partial_d) HIP_OK(hipFree(s->partial_d));
   s->partial_d = nullptr;
-  HIP_OK(hipMalloc(&s->partial_d, n_doubles * sizeof(double)));
+  HIP_OK(m3lb::device_alloc(s->device, &s->partial_d, n_doubles * sizeof(double)));
   s->partial_n = n_doubles;
   return M3LB_OK;
 }
@@ -207,7 +211,7 @@ int ensure_work(m3lb_solver* s, size_t bytes) {
   if (s->work_d) HIP_OK(hipFree(s->work_d));
   s->work_d = nullptr;
   s->work_n = 0;
-  HIP_OK(hipMalloc(&s->work_d, bytes));
+  HIP_OK(m3lb::device_alloc(s->device, &s->work_d, bytes));
   s->work_n = bytes;
   return M3LB_OK;
 }
@@ -358,11 +362,11 @@ double real_mul(const m3lb_solver* s, double a, double c) {
 
 // Re-uploads a small host vector into a device array of its size.
 template <class T>
-int upload(T*& dst, const std::vector<T>& src, hipStream_t st) {
+int upload(const m3lb_solver* s, T*& dst, const std::vector<T>& src) {
   free_dev(dst);
-  HIP_OK(hipMalloc(&dst, std::max<size_t>(1, src.size()) * sizeof(T)));
+  HIP_OK(m3lb::device_alloc(s->device, &dst, std::max<size_t>(1, src.size()) * sizeof(T)));
   if (!src.empty())
-    HIP_OK(hipMemcpyAsync(dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice, st));
+    HIP_OK(hipMemcpyAsync(dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice, s->stream));
   return M3LB_OK;
 }
 
@@ -501,13 +505,13 @@ int rebuild_plan(m3lb_solver* s) {
     }
     corners.push_back(q);
   }
-  int rc = upload(b.wlist_d, wlist, s->stream);
-  if (!rc) rc = upload(b.slist_d, spec, s->stream);
-  if (!rc) rc = upload(b.snap_nodes_d, snap_nodes, s->stream);
-  if (!rc) rc = upload(b.rd_d, rd, s->stream);
+  int rc = upload(s, b.wlist_d, wlist);
+  if (!rc) rc = upload(s, b.slist_d, spec);
+  if (!rc) rc = upload(s, b.snap_nodes_d, snap_nodes);
+  if (!rc) rc = upload(s, b.rd_d, rd);
   if (rc) return rc;
   free_dev(b.snap_d);
-  HIP_OK(hipMalloc(&b.snap_d, std::max<size_t>(1, snap_nodes.size()) * size_t(s->Q) *
+  HIP_OK(m3lb::device_alloc(s->device, &b.snap_d, std::max<size_t>(1, snap_nodes.size()) * size_t(s->Q) *
                                   size_t(s->ks->real_bytes)));
   SYNC_OK(s);
   b.dirty = false;
@@ -558,6 +562,7 @@ int sync(m3lb_solver* s) {
   return M3LB_OK;
 }
 
+bool give_back_alt(void* owner);
 int calibrate(m3lb_solver* s);
 int seed_calibrated(m3lb_solver* s, m3lb::SeedArgs a);
 
@@ -642,17 +647,17 @@ int m3lb_create(const m3lb_config* cfg, m3lb_solver** out) {
   if (hipEventCreate(&s->ev0) != hipSuccess || hipEventCreate(&s->ev1) != hipSuccess)
     return bail(fail(M3LB_EDEVICE, "hipEventCreate failed"));
   const size_t fbytes = s->stride * size_t(s->Q) * size_t(ks->elem_bytes);
-  if (hipMalloc(&s->f, fbytes) != hipSuccess)
+  if (m3lb::device_alloc(s->device, &s->f, fbytes) != hipSuccess)
     return bail(fail(M3LB_ENOMEM, "population array: hipMalloc of " + std::to_string(fbytes) + " bytes failed"));
   // Kokkos Views are zero-initialised; so is this.
   if (hipMemsetAsync(s->f, 0, fbytes, s->stream) != hipSuccess)
     return bail(fail(M3LB_EDEVICE, "hipMemsetAsync failed"));
-  if (hipMalloc(&s->flags_d, size_t(np)) != hipSuccess)
+  if (m3lb::device_alloc(s->device, &s->flags_d, size_t(np)) != hipSuccess)
     return bail(fail(M3LB_ENOMEM, "flags: hipMalloc failed"));
   if (cfg->forcing == M3LB_FORCE_FIELD) {
     // the per-node force starts at zero everywhere
     const size_t ffb = 3 * s->stride * size_t(ks->real_bytes);
-    if (hipMalloc(&s->ff_d, ffb) != hipSuccess)
+    if (m3lb::device_alloc(s->device, &s->ff_d, ffb) != hipSuccess)
       return bail(fail(M3LB_ENOMEM, "force field: hipMalloc failed"));
     if (hipMemsetAsync(s->ff_d, 0, ffb, s->stream) != hipSuccess)
       return bail(fail(M3LB_EDEVICE, "hipMemsetAsync failed"));
@@ -666,12 +671,14 @@ int m3lb_create(const m3lb_config* cfg, m3lb_solver** out) {
   if (hipMemcpyAsync(s->flags_d, s->flags_h.data(), size_t(np), hipMemcpyHostToDevice, s->stream) != hipSuccess)
     return bail(fail(M3LB_EDEVICE, "flags upload failed"));
   if (hipStreamSynchronize(s->stream) != hipSuccess) return bail(fail(M3LB_EDEVICE, "sync failed"));
+  if (ks->plane || ks->march) m3lb::spare_register({s->device, s, give_back_alt});
   *out = s;
   return M3LB_OK;
 }
 
 int m3lb_destroy(m3lb_solver* s) {
   if (!s) return M3LB_OK;
+  m3lb::spare_unregister(s);
   if (s->stream) hipStreamSynchronize(s->stream);
   if (s->f) hipFree(s->f);
   if (s->f_alt) hipFree(s->f_alt);
@@ -836,7 +843,9 @@ int launch_pair(m3lb_solver* s, const m3lb::StepArgs& a, int parity) {
       s->pair_sync = nullptr;
       s->pair_sync_n = 0;
     }
-    HIP_OK(hipMalloc(&s->pair_sync, size_t(words) * 4));
+    // (this call holds alt_mu, so not device_alloc)
+    HIP_OK(m3lb::device_alloc_plain(s->device, reinterpret_cast<void**>(&s->pair_sync),
+                                    size_t(words) * 4));
     HIP_OK(hipMemsetAsync(s->pair_sync, 0, size_t(words) * 4, s->stream));
     s->pair_sync_n = words;
   }
@@ -886,7 +895,22 @@ m3lb::PlanePlan plane_plan(const m3lb_solver* s, int left) {
   return m3lb::plane_rule(p, left);
 }
 
-// The second population array: allocated at the first pass, and given the
+// Frees the second array, for an allocation of any handle that found no memory
+// (device_memory.hpp) and where the handle's settings have no use for it.
+bool give_back_alt(void* owner) {
+  m3lb_solver* s = static_cast<m3lb_solver*>(owner);
+  std::lock_guard<std::mutex> l(s->alt_mu);
+  if (!s->f_alt) return false;
+  if (hipStreamSynchronize(s->stream) != hipSuccess) {  // a pass may still read it
+    (void)hipGetLastError();
+    return false;
+  }
+  (void)hipFree(s->f_alt);
+  s->f_alt = nullptr;
+  return true;
+}
+
+// The second population array (the caller holds alt_mu): allocated at the first pass, and given the
 // slots no moving node writes whenever those may have changed.  *have: false where
 // there is no room for it now; the steps of this call go another way, and the next
 // call asks again.
@@ -895,11 +919,8 @@ int ensure_alt(m3lb_solver* s, bool statics, bool* have) {
   const size_t bytes = size_t(s->stride) * size_t(s->Q) * size_t(s->ks->elem_bytes);
   if (!s->f_alt) {
     // at most a quarter of what is free: other boxes keep room of their own
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || bytes > free_b / 4 ||
-        hipMalloc(&s->f_alt, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      s->f_alt = nullptr;
+    if (bytes > m3lb::device_free_bytes(s->device) / 4 ||
+        m3lb::device_alloc_plain(s->device, &s->f_alt, bytes) != hipSuccess) {
       *have = false;
       return M3LB_OK;
     }
@@ -999,6 +1020,9 @@ int m3lb_set_step_fusion(m3lb_solver* s, int32_t mode, int32_t stripes, int32_t 
   s->pair_lag = lag;
   s->pair_bpc = blocks_per_cu;
   s->pair_group = group;
+  const bool tuned = stripes || lag || blocks_per_cu || group;
+  if (mode == M3LB_FUSION_OFF || (s->Q == 27 && (mode != M3LB_FUSION_AUTO || tuned)))
+    give_back_alt(s);
   return M3LB_OK;
 }
 
@@ -1030,7 +1054,7 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   m3lb::StepArgs a = step_args(s);
   if (store_macroscopic) {
     for (int k = 0; k < 4; ++k) {
-      if (!s->macro_d[k]) HIP_OK(hipMalloc(&s->macro_d[k], size_t(s->d.np) * size_t(s->ks->real_bytes)));
+      if (!s->macro_d[k]) HIP_OK(m3lb::device_alloc(s->device, &s->macro_d[k], size_t(s->d.np) * size_t(s->ks->real_bytes)));
     }
   }
   const unsigned rows_per_block = unsigned(m3lb::kBlock >> a.bx_log2);
@@ -1052,6 +1076,7 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   na.count = b.nsnap;
   na.out = b.snap_d;
   for (int q = 0; q < 27; ++q) na.inv_scale[q] = s->inv_scale[q];
+  std::lock_guard<std::mutex> alt_lock(s->alt_mu);
   const bool pairs = pair_eligible(s, a);
   m3lb::MarchPlan march = march_plan(s, a);
   // An even number of steps from an odd one costs the passes through LDS two single
@@ -1412,7 +1437,10 @@ extern "C" int m3lb_stream_probe(uint64_t bytes, int32_t nontemporal, int32_t re
   if (!best_ms || bytes < 16 || reps < 1) return fail(M3LB_EINVAL, "bad argument");
   const uint64_t n4 = bytes / 16;
   f4v* a = nullptr;
-  if (hipMalloc(&a, n4 * 16) != hipSuccess) return fail(M3LB_ENOMEM, "stream probe: hipMalloc failed");
+  int device = 0;
+  HIP_OK(hipGetDevice(&device));
+  if (m3lb::device_alloc(device, &a, n4 * 16) != hipSuccess)
+    return fail(M3LB_ENOMEM, "stream probe: hipMalloc failed");
   hipStream_t st = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int rc = M3LB_OK;
@@ -1644,16 +1672,16 @@ int m3lb_set_regularized_walls(m3lb_solver* s, const uint8_t* normals, const uin
   }
   b.wtab0 = b.wtab;
   b.has_corners = corners;
-  int rc = upload(b.nrm_d, b.nrm, s->stream);
-  if (!rc) rc = upload(b.tag_d, b.tag, s->stream);
-  if (!rc) rc = upload(b.unk_d, b.unk, s->stream);
-  if (!rc) rc = upload(b.ext_d, b.ext, s->stream);
-  if (!rc) rc = upload(b.onrm_d, b.onrm, s->stream);
-  if (!rc) rc = upload(b.don_d, b.don, s->stream);
-  if (!rc) rc = upload(b.wtab_d, b.wtab, s->stream);
+  int rc = upload(s, b.nrm_d, b.nrm);
+  if (!rc) rc = upload(s, b.tag_d, b.tag);
+  if (!rc) rc = upload(s, b.unk_d, b.unk);
+  if (!rc) rc = upload(s, b.ext_d, b.ext);
+  if (!rc) rc = upload(s, b.onrm_d, b.onrm);
+  if (!rc) rc = upload(s, b.don_d, b.don);
+  if (!rc) rc = upload(s, b.wtab_d, b.wtab);
   if (rc) return rc;
   if (!b.rho_d) {
-    HIP_OK(hipMalloc(&b.rho_d, np * size_t(s->ks->real_bytes)));
+    HIP_OK(m3lb::device_alloc(s->device, &b.rho_d, np * size_t(s->ks->real_bytes)));
     HIP_OK(hipMemsetAsync(b.rho_d, 0, np * size_t(s->ks->real_bytes), s->stream));
   }
   HIP_OK(hipMemcpyAsync(s->flags_d, s->flags_h.data(), np, hipMemcpyHostToDevice, s->stream));
@@ -1730,7 +1758,7 @@ int m3lb_set_wall_velocity_field(m3lb_solver* s, const double* ux, const double*
       }
   SYNC_OK(s);
   Boundaries& b = s->b;
-  if (!b.un_d) HIP_OK(hipMalloc(&b.un_d, h.size()));
+  if (!b.un_d) HIP_OK(m3lb::device_alloc(s->device, &b.un_d, h.size()));
   HIP_OK(hipMemcpy(b.un_d, h.data(), h.size(), hipMemcpyHostToDevice));
   b.un_on = true;
   b.un_scale = 1.0;
@@ -1763,11 +1791,11 @@ int m3lb_set_specular_walls(m3lb_solver* s, const uint8_t* normals) {
         b.spec_nrm[n] = normals[k];
         s->flags_h[n] = M3LB_SPECWALL;
       }
-  int rc = upload(b.spec_nrm_d, b.spec_nrm, s->stream);
+  int rc = upload(s, b.spec_nrm_d, b.spec_nrm);
   if (rc) return rc;
   if (!b.spec_faces_d) {
     b.spec_faces.assign(np, 0);
-    rc = upload(b.spec_faces_d, b.spec_faces, s->stream);
+    rc = upload(s, b.spec_faces_d, b.spec_faces);
     if (rc) return rc;
   }
   HIP_OK(hipMemcpyAsync(s->flags_d, s->flags_h.data(), np, hipMemcpyHostToDevice, s->stream));
@@ -1800,11 +1828,11 @@ int m3lb_set_specular_nodes(m3lb_solver* s, const uint8_t* faces) {
         b.spec_faces[n] = faces[k];
         s->flags_h[n] = M3LB_SPECNODE;
       }
-  int rc = upload(b.spec_faces_d, b.spec_faces, s->stream);
+  int rc = upload(s, b.spec_faces_d, b.spec_faces);
   if (rc) return rc;
   if (!b.spec_nrm_d) {
     b.spec_nrm.assign(np, 0);
-    rc = upload(b.spec_nrm_d, b.spec_nrm, s->stream);
+    rc = upload(s, b.spec_nrm_d, b.spec_nrm);
     if (rc) return rc;
   }
   HIP_OK(hipMemcpyAsync(s->flags_d, s->flags_h.data(), np, hipMemcpyHostToDevice, s->stream));
@@ -1920,6 +1948,7 @@ int m3lb_device_bytes(const m3lb_solver* s, uint64_t* bytes) {
   for (void* p : s->macro_d)
     if (p) b += uint64_t(s->d.np) * uint64_t(s->ks->real_bytes);
   b += s->partial_n * sizeof(double);
+  std::lock_guard<std::mutex> l(s->alt_mu);
   if (s->f_alt) b += s->stride * uint64_t(s->Q) * uint64_t(s->ks->elem_bytes);
   *bytes = b;
   return M3LB_OK;

@@ -79,3 +79,70 @@ def test_no_room_now_and_room_later(cfg):
         assert s.device_bytes() > 1.5 * base
         s.step(counts[2])
         assert np.array_equal(np.stack(s.compute_macroscopic()), want)
+
+
+@pytest.mark.parametrize("cfg", [PLANE, BOX], ids=["plane", "box"])
+def test_another_box_takes_the_array(cfg):
+    """A box that would not fit beside the second arrays of others is created, and
+    those step on without."""
+    counts = (4, 6, 5)
+    want = steps_of(cfg, counts)
+    with FluidSolver(cfg) as s:
+        base = init(s, cfg)
+        s.step(counts[0])
+        assert s.device_bytes() > 1.5 * base
+        with nearly_full(0.5 * base), FluidSolver(cfg) as other:
+            assert s.device_bytes() < 1.5 * base
+            init(other, cfg)
+            other.step(sum(counts))
+            s.step(counts[1])
+            assert s.device_bytes() < 1.5 * base
+            assert np.array_equal(np.stack(other.compute_macroscopic()), want)
+        s.step(counts[2])
+        assert s.device_bytes() > 1.5 * base
+        assert np.array_equal(np.stack(s.compute_macroscopic()), want)
+
+
+@pytest.mark.parametrize("cfg", [PLANE, BOX], ids=["plane", "box"])
+def test_settings_without_use_for_the_array_give_it_back(cfg):
+    with FluidSolver(cfg) as s:
+        base = init(s, cfg)
+        s.step(4)
+        assert s.device_bytes() > 1.5 * base
+        s.set_step_fusion(abi.FUSION_OFF)
+        assert s.device_bytes() < 1.5 * base
+        s.step(4)
+        s.set_step_fusion(abi.FUSION_AUTO)
+        s.step(4)
+        assert s.device_bytes() > 1.5 * base
+        if cfg.lattice == abi.D3Q27:
+            s.set_step_fusion(abi.FUSION_AUTO, stripes=8)
+            assert s.device_bytes() < 1.5 * base
+
+
+def test_array_taken_while_another_thread_steps():
+    """Allocations of one thread take the array of a box that another one steps."""
+    import threading
+    cfg, n = PLANE, 40
+    want = steps_of(cfg, [4] * n)
+    with FluidSolver(cfg) as s:
+        base = init(s, cfg)
+
+        def run():
+            for _ in range(n):
+                s.step(4)
+        with nearly_full(6 * base):
+            t = threading.Thread(target=run)
+            t.start()
+            for _ in range(6):
+                boxes = []
+                try:
+                    for _ in range(8):
+                        boxes.append(FluidSolver(cfg))
+                except RuntimeError:
+                    pass  # full: every spare array is taken by then
+                for b in boxes:
+                    b.close()
+            t.join(60)
+            assert not t.is_alive()
+        assert np.array_equal(np.stack(s.compute_macroscopic()), want)
