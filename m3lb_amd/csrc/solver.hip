@@ -1001,6 +1001,40 @@ int launch_march(m3lb_solver* s, const m3lb::StepArgs& a, const m3lb::MarchPlan&
   return M3LB_OK;
 }
 
+// The passes that a step call may use.
+struct Passes {
+  bool pairs = false;
+  m3lb::MarchPlan march;
+  m3lb::PlanePlan plane;  // of the first pass
+};
+
+// Chooses them for `nsteps` steps and has the second array ready (the caller holds
+// alt_mu, and the boundary plan is up to date).
+int choose_passes(m3lb_solver* s, const m3lb::StepArgs& a, int nsteps, bool store, Passes& ps) {
+  const int odd = int(s->t % 2), passable = nsteps - (store ? 1 : 0);
+  ps.pairs = pair_eligible(s, a);
+  ps.march = march_plan(s, a);
+  // An even number of steps from an odd one costs the passes through LDS two single
+  // steps, the passes in place none.  us per step, in place / single steps and
+  // LDS, D3Q27 CM: FP32 512^3 2 steps 4176 / 5341, 6 4180 / 4372, 8 4180 / 4234, 10
+  // 4180 / 4154, 20 4182 / 3992; 256^3 2 558 / 667, 8 550 / 549; FP64 256^3 2 1098 /
+  // 1384, 8 1087 / 1143, 10 1085 / 1119, 20 1079 / 1075 (on a card with 1295 in place
+  // 20 1086).
+  if (ps.march.on && ps.pairs && odd && passable % 2 == 0 && passable < 10) ps.march.on = false;
+  if (ps.march.on && passable - odd >= 2) {
+    const int rc = ensure_alt(s, s->geometry || s->d.hx || s->d.hy || s->d.hz, &ps.march.on);
+    if (rc) return rc;
+  }
+  ps.plane = plane_plan(s, passable - odd);
+  if (ps.plane.steps) {
+    bool have = false;
+    const int rc = ensure_alt(s, ps.plane.nodes != m3lb::kPlaneFluid, &have);
+    if (rc) return rc;
+    if (!have) ps.plane.steps = 0;
+  }
+  return M3LB_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1077,27 +1111,12 @@ int m3lb_step(m3lb_solver* s, int32_t nsteps, int32_t store_macroscopic) {
   na.out = b.snap_d;
   for (int q = 0; q < 27; ++q) na.inv_scale[q] = s->inv_scale[q];
   std::lock_guard<std::mutex> alt_lock(s->alt_mu);
-  const bool pairs = pair_eligible(s, a);
-  m3lb::MarchPlan march = march_plan(s, a);
-  // An even number of steps from an odd one costs the passes through LDS two single
-  // steps, the passes in place none.  us per step, in place / single steps and
-  // LDS, D3Q27 CM: FP32 512^3 2 steps 4176 / 5341, 6 4180 / 4372, 8 4180 / 4234, 10
-  // 4180 / 4154, 20 4182 / 3992; 256^3 2 558 / 667, 8 550 / 549; FP64 256^3 2 1098 /
-  // 1384, 8 1087 / 1143, 10 1085 / 1119, 20 1079 / 1075 (on a card with 1295 in place
-  // 20 1086).
-  const int passable = nsteps - (store_macroscopic ? 1 : 0);
-  if (march.on && pairs && s->t % 2 == 1 && passable % 2 == 0 && passable < 10) march.on = false;
-  if (march.on && passable - int(s->t % 2) >= 2) {
-    const int rc = ensure_alt(s, s->geometry || s->d.hx || s->d.hy || s->d.hz, &march.on);
-    if (rc) return rc;
-  }
-  m3lb::PlanePlan plane = plane_plan(s, passable - int(s->t % 2));
-  if (plane.steps) {
-    bool have = false;
-    const int rc = ensure_alt(s, plane.nodes != m3lb::kPlaneFluid, &have);
-    if (rc) return rc;
-    if (!have) plane.steps = 0;
-  }
+  Passes ps;
+  const int prc = choose_passes(s, a, nsteps, store_macroscopic != 0, ps);
+  if (prc) return prc;
+  const bool pairs = ps.pairs;
+  const m3lb::MarchPlan& march = ps.march;
+  m3lb::PlanePlan plane = ps.plane;
   for (int k = 0; k < nsteps; ++k) {
     const bool last = k == nsteps - 1;
     // the plane passes: even numbers of steps from an even one (never the
@@ -1165,6 +1184,12 @@ int m3lb_time_steps(m3lb_solver* s, int32_t nsteps, double* ms) {
   if (!s || !ms) return fail(M3LB_EINVAL, "null argument");
   if (s->b.dirty) {  // the boundary plan is host work: keep it out of the timing
     const int rc = rebuild_plan(s);
+    if (rc) return rc;
+  }
+  if (nsteps > 0) {  // and the second array, with what it has to hold before the first pass
+    std::lock_guard<std::mutex> l(s->alt_mu);
+    Passes ps;
+    const int rc = choose_passes(s, step_args(s), nsteps, false, ps);
     if (rc) return rc;
   }
   HIP_OK(hipEventRecord(s->ev0, s->stream));
