@@ -55,6 +55,7 @@ def gpu_leg(D, steps, warmup, dtype, op, seed=3, field=None, fusion=None):
     cfg, u0 = taylor_green_config(abi, D, dtype, op)
     t0 = time.time()
     s = FluidSolver(cfg)
+    own = s.device_bytes()
     if fusion is not None:
         s.set_step_fusion(fusion)
     if field is None:
@@ -66,6 +67,7 @@ def gpu_leg(D, steps, warmup, dtype, op, seed=3, field=None, fusion=None):
     ms = s.time_steps(steps)
     m1 = s.total_mass()
     e, w, finite = s.energy_enstrophy()
+    two_arrays = s.device_bytes() > 1.5 * own
     s.close()
     nodes = D ** 3
     sec = ms / 1e3
@@ -73,7 +75,31 @@ def gpu_leg(D, steps, warmup, dtype, op, seed=3, field=None, fusion=None):
     per_launch_s = sec / steps
     achieved = bytes_per_node(abi, dtype) * nodes / per_launch_s / 1e9
     return dict(mlups=mlups, ms=ms, ms_per_step=ms / steps, achieved_gbs=achieved,
-                mass_drift=abs(m1 - m0) / m0, finite=finite)
+                mass_drift=abs(m1 - m0) / m0, finite=finite, two_arrays=two_arrays)
+
+
+def stored_traffic(fusion, two_arrays, build, profiles=os.path.join(ROOT, "profiles")):
+    """Bytes per step between the L2 caches and the memory fabric for the 512^3 FP32 CM
+    workload, and where they come from: the committed rocprofv3 --pmc summary of the
+    pass that ran (FETCH_SIZE + WRITE_SIZE of one two-step pass, calibrated on a copy
+    kernel, halved), used only while the loaded library holds the kernels it was
+    measured on.  The pass through LDS writes a second array; without one, and with
+    fusion on, the pass in place ran; with fusion off none did.  These counters see
+    requests that the memory-side 256 MB cache serves as well as those that reach
+    HBM."""
+    if fusion == "off":
+        return None, None
+    name = "k_march" if fusion == "auto" and two_arrays else "k_pair"
+    path = os.path.join(profiles, name + "_cm_f32_512cubed_traffic.json")
+    if not os.path.exists(path):
+        return None, None
+    with open(path) as fh:
+        tr = json.load(fh)
+    if tr.get("build_id") != build:
+        return None, (f"null: the stored count was taken on build {tr.get('build_id')}, "
+                      f"the loaded library is build {build}")
+    return (tr["traffic_bytes"],
+            f"{tr['source']} (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE; build {build})")
 
 
 def host_cpu():
@@ -501,24 +527,10 @@ def main():
         f"nontemporal {ceil['nontemporal']:.0f} GB/s; step kernel at "
         f"{r['achieved_gbs'] / best_ceiling:.3f} of the better")
 
-    # Bytes per step between the L2 caches and the memory fabric, from the
-    # committed rocprofv3 --pmc summary of this exact workload (FETCH_SIZE +
-    # WRITE_SIZE of one two-step pass, calibrated on a copy kernel, halved),
-    # used only while the loaded library holds the kernels it was measured on.
-    # These counters see requests that the memory-side 256 MB cache serves as
-    # well as those that reach HBM.
-    traffic, traffic_src = None, None
-    tj = os.path.join(ROOT, "profiles", "k_march_cm_f32_512cubed_traffic.json")
     build = solver.kernel_build_id()
-    if args.size == 512 and args.dtype == "f32" and args.fusion != "off" and os.path.exists(tj):
-        with open(tj) as fh:
-            tr = json.load(fh)
-        if tr.get("build_id") == build:
-            traffic = tr["traffic_bytes"]
-            traffic_src = f"{tr['source']} (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE; build {build})"
-        else:
-            traffic_src = (f"null: the stored count was taken on build {tr.get('build_id')}, "
-                           f"the loaded library is build {build}")
+    traffic, traffic_src = None, None
+    if args.size == 512 and args.dtype == "f32":
+        traffic, traffic_src = stored_traffic(args.fusion, r["two_arrays"], build)
 
     # the same workload with E2M13 storage (108 B per node-step), run for
     # 2000 steps beside the same run with FP64 storage: rate and error

@@ -41,3 +41,25 @@ def test_cpu_baseline_uses_every_core_of_the_job(monkeypatch):
     assert bench.cpu_threads() == 1
     monkeypatch.setenv("OMP_NUM_THREADS", str(usable + 5))
     assert bench.cpu_threads() == usable
+
+
+def test_traffic_is_that_of_the_pass_that_ran(tmp_path):
+    """The stored byte counts are of one pass each: through LDS (a second array),
+    in place (one array, or fusion on); none with fusion off or on another build."""
+    import json
+
+    sys.path.insert(0, ROOT)
+    import bench
+    for name, n in (("k_march", 17), ("k_pair", 29)):
+        (tmp_path / f"{name}_cm_f32_512cubed_traffic.json").write_text(
+            json.dumps({"build_id": "abc", "traffic_bytes": n, "source": name}))
+
+    def count(fusion, two_arrays, build="abc"):
+        return bench.stored_traffic(fusion, two_arrays, build, str(tmp_path))[0]
+    assert count("auto", True) == 17
+    assert count("auto", False) == 29
+    assert count("on", False) == 29
+    assert count("on", True) == 29
+    assert count("off", False) is None
+    assert count("auto", True, "other") is None
+    assert "abc" in bench.stored_traffic("auto", True, "other", str(tmp_path))[1]
