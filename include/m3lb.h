@@ -141,9 +141,11 @@ typedef struct m3lb_solver m3lb_solver;
  * out = {nx, ny, nz, hx, hy, hz, sx, sy, sz, n_padded}. */
 int m3lb_domain(const m3lb_config* cfg, int64_t out[10]);
 
-/* FluidSolver(Domain, Collision) (FluidSolver.hpp:42-69): allocates the one
- * in-place population array, the flag array (halo Excluded, interior Fluid)
- * and the macroscopic arrays on the current HIP device. */
+/* FluidSolver(Domain, Collision) (FluidSolver.hpp:42-69): allocates the
+ * in-place population array and the flag array (halo Excluded, interior Fluid)
+ * on the current HIP device, the handle's from then on.  The macroscopic arrays come
+ * with the first step that stores them; a second population array, of the size of
+ * the first, comes with the first pass that writes one (m3lb_set_step_fusion). */
 int m3lb_create(const m3lb_config* cfg, m3lb_solver** out);
 int m3lb_destroy(m3lb_solver* s);
 const char* m3lb_last_error(void);
@@ -297,8 +299,9 @@ int m3lb_set_scales(m3lb_solver* s, const double* scales_q);
 int m3lb_calibrate_scales(m3lb_solver* s);
 
 /* Runs nsteps steps bracketed by HIP events recorded on the handle's stream
- * and returns the elapsed milliseconds.  Used by the benchmark.  No
- * counterpart in the reference. */
+ * and returns the elapsed milliseconds, without the boundary plan and the second
+ * array's allocation and first copy, which are done before.  Used by the
+ * benchmark.  No counterpart in the reference. */
 int m3lb_time_steps(m3lb_solver* s, int32_t nsteps, double* ms);
 
 /* Order in which the step kernel's tiles are assigned to the GPU's 8 XCDs:
@@ -317,17 +320,34 @@ int m3lb_set_tile_order(m3lb_solver* s, int32_t run);
 enum { M3LB_CACHE_AUTO = 0, M3LB_CACHE_STREAM = 1, M3LB_CACHE_PLAIN = 2 };
 int m3lb_set_cache_policy(m3lb_solver* s, int32_t policy);
 
-/* Two steps in one pass over the population array.  By default the steps of an
- * FP32 or FP64 D3Q27 box beyond the last-level cache (CM, MRT, BGK with the
- * product equilibrium; no per-node force) run through LDS into a
- * second array of the same size (held from the first pass on, where a quarter of
- * the free device memory has room for it); the values below tune the pass used
- * where that one does not apply or any of them is set.  There step t+1 follows step t
+/* Several steps in one pass over the population array.  Every pass below leaves the
+ * bits that one launch per step leaves.
+ *
+ * D2Q9 boxes without a per-node force, outlets and specular cells take 2 to 8 steps
+ * per launch in LDS, regularised walls included, wherever that is the faster way
+ * (by the box's size and shape, storage and walls), under AUTO and under ON;
+ * m3lb_fused_passes does not count these launches, and tile order and cache policy
+ * do not apply to them.
+ *
+ * FP32 and FP64 D3Q27 boxes beyond the last-level cache (CM, MRT, BGK with the
+ * product equilibrium; no per-node force, no walls) take two steps per pass through
+ * LDS under AUTO with no tuning value set.
+ *
+ * Both write a second population array of the same size.  It is allocated on the
+ * handle's device at the first such pass where it takes no more than a quarter of
+ * the free memory; otherwise the steps of that call go another way and the next
+ * call asks again.  An allocation of this library, of any handle, that finds no
+ * memory takes the idle second arrays of its device back first; other programs
+ * and libraries see the memory as taken.  M3LB_FUSION_OFF gives the array back, and
+ * for D3Q27 ON and the tuning values too.
+ *
+ * The values below tune the pass of D3Q27 boxes in place, used where the one
+ * through LDS does not apply, for even numbers of steps below ten from an odd step,
+ * under ON, and where any value is set.  There step t+1 follows step t
  * a few z-planes behind inside one persistent launch, so that it reads step
  * t's output from the caches, and a short second launch finishes the rows
  * whose neighbours another stripe of the box updates: a pair of steps then
- * moves about the HBM bytes of one.  The result is bit-identical to one launch
- * per step.  No counterpart in the reference.
+ * moves about the HBM bytes of one.  No counterpart in the reference.
  *   mode  M3LB_FUSION_AUTO (default): pair the steps of FP32 and FP64 boxes
  *         whose population array exceeds the 256 MB last-level cache (the
  *         16-bit forms run faster one launch per step);
@@ -353,7 +373,8 @@ int m3lb_set_step_fusion(m3lb_solver* s, int32_t mode, int32_t stripes, int32_t 
  * that array and race; one call at a time per GPU. */
 int m3lb_totals_static(m3lb_solver* s, double out[4]);
 
-/* Pairs of steps the handle has run as one pass since creation. */
+/* Pairs of steps of a D3Q27 box that the handle has run as one pass, of either
+ * kind, since creation. */
 int m3lb_fused_passes(const m3lb_solver* s, uint64_t* passes);
 /* Failure-path test hook: with on != 0 every wait of a two-step pass is made
  * unsatisfiable and gives up after a few polls, so the pass drains at once
@@ -385,7 +406,9 @@ int m3lb_stream_probe(uint64_t bytes, int32_t nontemporal, int32_t reps, double*
  * counterpart in the reference. */
 const char* m3lb_kernel_build_id(void);
 
-/* Device bytes held by the handle (populations + flags + macroscopic). */
+/* Device bytes held by the handle: populations, the second array while it is held,
+ * flags, macroscopic arrays and reduction partials.  Not counted: boundary data and
+ * the scratch of loads and energies, of which at most 64 MB is kept between calls. */
 int m3lb_device_bytes(const m3lb_solver* s, uint64_t* bytes);
 /* initialize_field with the Taylor-Green vortex of
  * validation/tgv3d_bench.cpp:79-90 evaluated on the device: w = 0,

@@ -361,7 +361,7 @@ class FluidSolver:
         _check(self.L.m3lb_calibrate_scales(self.h))
 
     def set_step_fusion(self, mode, stripes=0, lag=0, blocks_per_cu=0, group=0):
-        """m3lb_set_step_fusion: pair steps in one pass (bit-identical results)."""
+        """m3lb_set_step_fusion: several steps in one pass (bit-identical results)."""
         _check(self.L.m3lb_set_step_fusion(self.h, int(mode), int(stripes), int(lag),
                                            int(blocks_per_cu), int(group)))
 
@@ -372,7 +372,7 @@ class FluidSolver:
         return out
 
     def fused_passes(self):
-        """m3lb_fused_passes: pairs of steps run as one pass so far."""
+        """m3lb_fused_passes: pairs of D3Q27 steps run as one pass so far."""
         n = ctypes.c_uint64()
         _check(self.L.m3lb_fused_passes(self.h, ctypes.byref(n)))
         return n.value
